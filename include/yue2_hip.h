@@ -238,8 +238,9 @@ int32_t yue2_hip_cache_load(Yue2Cache *c, const float *key, const float *value, 
 int32_t yue2_hip_cache_export(const Yue2Cache *c, float *key, float *value, int32_t start, int32_t n,
                               int32_t stride);
 
-/* Model::forward_phase (src/model.rs:465-477): run n ids through the model,
- * appending to the cache; write the logits of the last row (vocab_size f32,
+/* Model::forward_phase (src/model.rs:465-477): run n ids through the model
+ * (many at once through multi-row kernels that keep the decode order, few
+ * token by token: the same bits), appending to the cache; write the logits of the last row (vocab_size f32,
  * BF16-exact) when logits != NULL. */
 int32_t yue2_hip_forward(Yue2Model *m, Yue2Cache *c, const int32_t *ids, int32_t n,
                          int32_t phase, float *logits);
@@ -446,8 +447,8 @@ int32_t yue2_hip_model_set_step_kernel(Yue2Model *m, int32_t on);
  * 3B-class prompt in ~20 ms, agreeing with the decode-order prefill within
  * its stated tolerance, not bit for bit -- as the reference's GPU prefill,
  * MPS GEMMs, src/tensor.rs:991-993, differs from its CPU path) or, the
- * default, the decode-order prefill (bit-exact, ~650 tokens/s).  Returns the
- * setting now in force (1 or 0). */
+ * default, the decode-order prefill (bit-exact, ~150 ms for that prompt).
+ * Returns the setting now in force (1 or 0). */
 int32_t yue2_hip_model_set_prefill(Yue2Model *m, int32_t mfma);
 /* Diagnostics: advance the launch sequence of the model's own workspace (the
  * one yue2_hip_forward uses) by `add`, as if that many step-kernel launches

@@ -1,0 +1,98 @@
+"""The multi-row decode-order forward (rows.hip) against token steps.
+
+Model::forward_phase over n ids (src/model.rs:469-477) is what n calls of one
+id compute, bit for bit: the logits of the last row and every cached key and
+value.  One-id calls run the token step, which the other tests pin to the
+oracle; the first case here is pinned to the oracle directly.  Sizes sit at
+the edges of the kernels: 16 queries per wave, 32-row tiles, 64-key blocks,
+128 rows per attention workgroup, contraction lengths of fewer than eight
+64-element lines and of a count that eight does not divide, the 256-block
+limit past which blocks are added in pairs."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from yue2_rs_amd import synthetic
+from yue2_rs_amd.api import Config
+import yue2_rs_amd as y2
+
+from helpers import bits, rb
+
+pytestmark = pytest.mark.gpu
+
+
+def _config(hidden, heads, kv_heads, head_dim, inter, layers=2, vocab=4096):
+    return Config(hidden_size=hidden, num_hidden_layers=layers, num_attention_heads=heads,
+                  num_key_value_heads=kv_heads, head_dim=head_dim, intermediate_size=inter, vocab_size=vocab,
+                  max_position_embeddings=24576, rms_norm_eps=1e-6, rope_theta=10000.0)
+
+
+SHAPES = {
+    "d64": _config(1024, 16, 4, 64, 2816),          # 16, 16, 44 lines
+    "d128": _config(1280, 10, 5, 128, 3456),        # 20, 20, 54 lines
+    "small": _config(320, 4, 2, 64, 448),           # 5, 4, 7 lines
+    "wide": _config(4096, 32, 8, 128, 14336, layers=1),
+}
+
+
+@pytest.fixture(scope="module", params=list(SHAPES), ids=list(SHAPES))
+def shape(request, gpu, oracle_threads):
+    ck = synthetic.checkpoint(SHAPES[request.param], seed=5)
+    gm = y2.Model.open(ck)
+    yield request.param, ck, gm
+    gm.close()
+
+
+def _filled(gm, context, capacity, seed):
+    c, cfg = y2.Cache(gm, capacity), gm.config
+    if context:
+        rng = np.random.default_rng(seed)
+        shape = (cfg.num_hidden_layers, context, cfg.num_key_value_heads * cfg.head_dim)
+        c.load(rb(rng.standard_normal(shape)), rb(rng.standard_normal(shape)), context)
+    return c
+
+
+def _check(gm, context, n, seed, phase=0):
+    cap = context + n + 3
+    ids = synthetic.prompt(n + 1, gm.config.vocab_size, seed)
+    a, b = _filled(gm, context, cap, seed), _filled(gm, context, cap, seed)
+    print(f"context {context}, {n} ids", flush=True)
+    got = gm.forward_phase(ids[:n], a, phase)
+    for t in ids[:n]:
+        want = gm.forward_phase([t], b, phase)
+    assert a.length == b.length == context + n
+    assert np.array_equal(bits(got), bits(want)), "last row's logits differ"
+    for x, y in zip(a.export(context, n), b.export(context, n)):
+        assert np.array_equal(bits(x), bits(y)), "cached rows differ"
+    # and a step on top of the multi-row cache
+    assert np.array_equal(bits(gm.forward(ids[n:], a)), bits(gm.forward(ids[n:], b)))
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("n", [4, 15, 16, 17, 32, 33, 64, 65, 129, 300])
+def test_prompt_equals_token_steps(shape, n):
+    _check(shape[2], 0, n, seed=n)
+
+
+@pytest.mark.parametrize("context,n", [(1, 4), (63, 5), (100, 37), (500, 130)])
+def test_append_equals_token_steps(shape, context, n):
+    _check(shape[2], context, n, seed=context + n)
+
+
+@pytest.mark.parametrize("context,n", [(16200, 121), (16255, 130), (16256, 129), (16400, 130)])
+def test_long_append_equals_token_steps(shape, context, n):
+    if shape[0] in ("d64", "d128"):
+        _check(shape[2], context, n, seed=context + n)
+
+
+def test_prompt_equals_oracle(gpu, oracle_threads):
+    ck = synthetic.checkpoint(SHAPES["d64"], seed=6)
+    gm, om = y2.Model.open(ck), O.Model(ck)
+    ids = synthetic.prompt(83, gm.config.vocab_size, 4)
+    oc = O.Cache(om, 90)
+    cache, got = gm.prefill_phase(ids, 90)
+    assert np.array_equal(bits(got), bits(om.forward(ids, oc)))
+    for x, y in zip(cache.export(), oc.arrays()):
+        assert np.array_equal(bits(x), bits(y[:, :83]))
+    gm.close()

@@ -36,6 +36,9 @@ constexpr int kGemmTK = 64;
 
 hipError_t launch_gemm(hipStream_t s, int epi, const GemmArgs& g);
 
+// x[r] = the embedding row of ids[r] as f32 for r < rows (ids in range).
+hipError_t launch_embed_rows(hipStream_t s, const uint16_t* embed, const int32_t* ids, float* x, int rows, int H);
+
 // out[r] = RMSNorm(x[r]) as BF16 for r < rows (x row stride H).
 hipError_t launch_norm_rows(hipStream_t s, const float* x, const float* gamma, uint16_t* out, int rows, int H,
                             float eps);

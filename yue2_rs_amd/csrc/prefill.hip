@@ -555,6 +555,12 @@ __global__ __launch_bounds__(kFlashThreads, 2) void flash_prefill_kernel(const F
     }
 }
 
+hipError_t launch_embed_rows(hipStream_t s, const uint16_t* embed, const int32_t* ids, float* x, int rows, int H) {
+    if (rows < 1) return hipSuccess;
+    embed_rows_kernel<<<rows, kRowThreads, 0, s>>>(embed, ids, x, H);
+    return hipGetLastError();
+}
+
 hipError_t launch_norm_rows(hipStream_t s, const float* x, const float* gamma, uint16_t* out, int rows, int H,
                             float eps) {
     if (rows < 1) return hipSuccess;
@@ -635,7 +641,8 @@ int run_prefill(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase
     const float eps = cf.rms_norm_eps;
     for (int p0 = 0; p0 < n; p0 += R) {
         const int rows = std::min(R, n - p0);
-        embed_rows_kernel<<<rows, kRowThreads, 0, s>>>(m->embed, b.ids + p0, b.x, H);
+        if ((e = launch_embed_rows(s, m->embed, b.ids + p0, b.x, rows, H)) != hipSuccess)
+            return hip_fail(e, "prefill embedding");
         for (int l = 0; l < cf.num_hidden_layers; ++l) {
             const LayerDev& L = m->layers[l];
             if ((e = launch_norm_rows(s, b.x, L.in_norm, b.h, rows, H, eps)) != hipSuccess)

@@ -17,6 +17,7 @@
 
 #include "../../include/yue2_hip.h"
 #include "kernels.h"
+#include "rows.h"
 #include "runtime.h"
 #include "step.h"
 #include "y2_math.h"
@@ -746,8 +747,9 @@ extern "C" int32_t yue2_hip_cache_export(const Yue2Cache* c, float* key, float* 
     return YUE2_OK;
 }
 
-// Model::forward_phase: token-by-token through the decode-order kernels, so a
-// prefill produces bit-for-bit the cache a sequence of decode steps would.
+// Model::forward_phase: many ids at once through the multi-row decode-order
+// kernels (rows.hip) where they are the faster way, else token by token; both
+// give bit for bit the cache a sequence of decode steps would.
 extern "C" int32_t yue2_hip_forward(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int32_t n,
                                     int32_t phase, float* logits) {
     std::lock_guard<std::recursive_mutex> guard(library_lock());
@@ -760,6 +762,16 @@ extern "C" int32_t yue2_hip_forward(Yue2Model* m, Yue2Cache* c, const int32_t* i
             return fail(YUE2_ERR_TOKEN, "Token outside model vocabulary");
     const int blocks = (c->capacity + kBlockKeys - 1) / kBlockKeys;
     if (int rc = m->ws.ensure(1, blocks, m->c)) return rc;
+    if (rows_supported(m, c->length, n)) {
+        const int rc = run_rows(m, c, ids, n, phase, logits != nullptr);
+        if (rc < 0) return rc;
+        if (rc == 0) {
+            c->length += n;
+            if (!logits) return YUE2_OK;
+            const hipError_t e = hipMemcpy(logits, m->ws.logits, sizeof(float) * m->c.vocab_size, hipMemcpyDeviceToHost);
+            return e == hipSuccess ? YUE2_OK : hip_fail(e, "logits readback");
+        }
+    }
     if (m->step_kernel)
         if (int rc = prepare_step(m, m->ws); rc < 0) return rc;
     KvView kv{};
