@@ -144,8 +144,8 @@ extern "C" Yue2Decoder* yue2_hip_decoder_new(Yue2Model* m, Yue2Cache* cond, Yue2
     d->need_rng = sampling && sampling->temperature != 0.0f;
     hipError_t e = hipSuccess;
     if (rc == YUE2_OK && d->need_rng) {
-        e = hipMalloc(&d->mt, sizeof(MtState));
-        if (e == hipSuccess) e = hipMalloc(&d->streams, sizeof(uint32_t) * 4 * (size_t)V);
+        e = device_malloc(&d->mt, sizeof(MtState));
+        if (e == hipSuccess) e = device_malloc(&d->streams, sizeof(uint32_t) * 4 * (size_t)V);
         if (e == hipSuccess) {
             MtState host;
             mt_seed(&host, seed);
@@ -157,15 +157,15 @@ extern "C" Yue2Decoder* yue2_hip_decoder_new(Yue2Model* m, Yue2Cache* cond, Yue2
     const int list = choose_list_len(V, mode, temp, sampling ? sampling->top_k : 1);
     const int chunks = (V + kChooseChunk - 1) / kChooseChunk;
     if (rc == YUE2_OK && e == hipSuccess && list > 0)
-        e = hipMalloc(&d->cand, sizeof(uint64_t) * (size_t)chunks * list + sizeof(int2) * chunks);
-    if (rc == YUE2_OK && e == hipSuccess && d->need_rng) e = hipMalloc(&d->big, survivor_bytes(V));
+        e = device_malloc(&d->cand, sizeof(uint64_t) * (size_t)chunks * list + sizeof(int2) * chunks);
+    if (rc == YUE2_OK && e == hipSuccess && d->need_rng) e = device_malloc(&d->big, survivor_bytes(V));
     const int flist = (mode == 0 || temp == 0.0f) ? 1 : (sampling ? sampling->top_k : 1);
     int head_lo, head_n, head_stop;
     head_rows(phase, V, &head_lo, &head_n, &head_stop);
     d->fused = m->step_kernel &&
                fused_sampler_supported(m->c, d->rows, m->cus, mode, temp, sampling ? sampling->top_k : 1, head_n);
     if (rc == YUE2_OK && e == hipSuccess && d->fused)
-        e = hipMalloc(&d->fcand, sizeof(uint64_t) * (size_t)(m->cus - 1) * flist);
+        e = device_malloc(&d->fcand, sizeof(uint64_t) * (size_t)(m->cus - 1) * flist);
     if (rc == YUE2_OK && e == hipSuccess) e = hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking);
     if (rc == YUE2_OK && e == hipSuccess) e = hipEventCreateWithFlags(&d->fork, hipEventDisableTiming);
     if (rc == YUE2_OK && e == hipSuccess) e = hipEventCreateWithFlags(&d->join, hipEventDisableTiming);
@@ -631,27 +631,6 @@ static int choose_check(const float* logits, int32_t vocab, const Yue2Sampling* 
     return YUE2_OK;
 }
 
-// sampling::choose (src/sampling.rs:103-215) for one row of logits.
-extern "C" int32_t yue2_hip_choose(const float* logits, int32_t vocab, const Yue2Sampling* sampling,
-                                   const int32_t* history, int32_t history_len, int32_t step,
-                                   int32_t phase, int32_t legacy, const uint32_t* draws,
-                                   int32_t* id) {
-    std::lock_guard<std::recursive_mutex> guard(library_lock());
-    if (int rc = choose_check(logits, vocab, sampling, history, history_len, step, phase, draws, id)) return rc;
-    const ChooseLayout L = choose_layout(vocab, sampling, history_len);
-    char* p = nullptr;
-    hipError_t e = hipMalloc(&p, L.total);
-    if (e != hipSuccess) return hip_fail(e, "hipMalloc(choose)");
-    hipStream_t s = nullptr;
-    e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    int rc = e == hipSuccess ? choose_run(p, L, s, logits, vocab, sampling, history, history_len, step, phase,
-                                          legacy, draws, id)
-                             : hip_fail(e, "hipStreamCreate(choose)");
-    if (s) (void)hipStreamDestroy(s);
-    (void)hipFree(p);
-    return rc;
-}
-
 // ---- choose() without allocation -------------------------------------------
 //
 // The scratch of yue2_hip_choose_noalloc: one region per device, laid out by
@@ -679,6 +658,43 @@ static int noalloc_scratch(char** out) {
     }
     *out = g_scratch_dev[dev];
     return YUE2_OK;
+}
+
+// The stream of yue2_hip_choose on the current device, made on its first use
+// and kept (null: it could not be made).
+static hipStream_t choose_stream() {
+    static hipStream_t streams[kNoAllocDevices];
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kNoAllocDevices) return nullptr;
+    if (!streams[dev] && hipStreamCreateWithFlags(&streams[dev], hipStreamNonBlocking) != hipSuccess)
+        streams[dev] = nullptr;
+    return streams[dev];
+}
+
+// sampling::choose (src/sampling.rs:103-215) for one row of logits.  A call
+// that fits the scratch array of the allocation-free entry runs there (the
+// library lock serialises its users and every call ends with its stream
+// idle), on a stream of its own that is kept: an allocation, a stream and
+// their frees were 70 of a call's 200 us at 84000 entries.
+extern "C" int32_t yue2_hip_choose(const float* logits, int32_t vocab, const Yue2Sampling* sampling,
+                                   const int32_t* history, int32_t history_len, int32_t step,
+                                   int32_t phase, int32_t legacy, const uint32_t* draws,
+                                   int32_t* id) {
+    std::lock_guard<std::recursive_mutex> guard(library_lock());
+    if (int rc = choose_check(logits, vocab, sampling, history, history_len, step, phase, draws, id)) return rc;
+    const ChooseLayout L = choose_layout(vocab, sampling, history_len);
+    hipStream_t s = choose_stream();
+    if (!s) return fail(YUE2_ERR_DEVICE, "hipStreamCreate(choose)");
+    char* p = nullptr;
+    if (L.total <= kNoAllocScratchBytes) {
+        if (int rc = noalloc_scratch(&p)) return rc;
+        return choose_run(p, L, s, logits, vocab, sampling, history, history_len, step, phase, legacy, draws, id);
+    }
+    hipError_t e = device_malloc(&p, L.total);
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc(choose)");
+    const int rc = choose_run(p, L, s, logits, vocab, sampling, history, history_len, step, phase, legacy, draws, id);
+    (void)hipFree(p);
+    return rc;
 }
 
 extern "C" int32_t yue2_hip_choose_noalloc(const float* logits, int32_t vocab, const Yue2Sampling* sampling,

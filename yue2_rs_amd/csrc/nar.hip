@@ -99,7 +99,7 @@ extern "C" int32_t yue2_hip_nar_load(Yue2Model* m, const Yue2NarWeights* w) {
     if (m->nar.block) (void)hipFree(m->nar.block);
     m->nar = NarDev{};
     void* block = nullptr;
-    hipError_t e = hipMalloc(&block, cv.offset);
+    hipError_t e = device_malloc(&block, cv.offset);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(NAR weights)");
     char* base = static_cast<char*>(block);
     NarDev& n = m->nar;
@@ -217,10 +217,9 @@ extern "C" int32_t yue2_hip_velocity(Yue2Model* m, const Yue2Cache* c, const flo
     const size_t o_att = cv.take<uint16_t>((size_t)n * qw), o_act = cv.take<uint16_t>((size_t)n * I);
     const size_t o_kv = cv.take<uint16_t>((size_t)cf.num_hidden_layers * 2 * Hkv * n * D);
     const size_t o_out = cv.take<float>((size_t)frames * Lat);
-    void* block = nullptr;
-    hipError_t e = hipMalloc(&block, cv.offset);
+    hipError_t e = m->scratch.ensure(cv.offset);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(NAR buffers)");
-    char* base = static_cast<char*>(block);
+    char* base = m->scratch.p;
     uint16_t* d_pad = reinterpret_cast<uint16_t*>(base + o_pad);
     uint16_t* d_sin = reinterpret_cast<uint16_t*>(base + o_sin);
     uint16_t* t0 = reinterpret_cast<uint16_t*>(base + o_t0);
@@ -282,7 +281,7 @@ extern "C" int32_t yue2_hip_velocity(Yue2Model* m, const Yue2Cache* c, const flo
     };
     const int rc = run();
     (void)hipStreamSynchronize(s);
-    (void)hipFree(block);
+    m->scratch.trim();
     return rc;
 }
 

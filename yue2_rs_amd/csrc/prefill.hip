@@ -600,13 +600,9 @@ namespace {
 constexpr int kPrefillChunk = 24576;
 
 struct PrefillBuffers {
-    void* block = nullptr;
-    float *x = nullptr, *qkv = nullptr, *logits_row = nullptr;
+    float *x = nullptr, *qkv = nullptr;
     uint16_t *h = nullptr, *q = nullptr, *att = nullptr, *act = nullptr;
     int32_t* ids = nullptr;
-    ~PrefillBuffers() {
-        if (block) (void)hipFree(block);
-    }
 };
 
 int run_prefill(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, float* logits) {
@@ -625,9 +621,9 @@ int run_prefill(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase
     const size_t o_h = take(2 * (size_t)R * std::max(H, I)), o_q = take(2 * (size_t)R * qw);
     const size_t o_att = take(2 * (size_t)R * qw), o_act = take(2 * (size_t)R * I);
     const size_t o_ids = take(sizeof(int32_t) * n);
-    hipError_t e = hipMalloc(&b.block, at);
+    hipError_t e = m->scratch.ensure(at);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(prefill buffers)");
-    char* p = static_cast<char*>(b.block);
+    char* p = m->scratch.p;
     b.x = reinterpret_cast<float*>(p + o_x);
     b.qkv = reinterpret_cast<float*>(p + o_qkv);
     b.h = reinterpret_cast<uint16_t*>(p + o_h);
@@ -697,7 +693,10 @@ extern "C" int32_t yue2_hip_prefill_mfma(Yue2Model* m, Yue2Cache* c, const int32
         (cf.num_attention_heads * cf.head_dim) % kGemmTK)
         return fail(YUE2_ERR_ARG, "shape without an MFMA prefill");
     if (int rc = m->ws.ensure(1, (c->capacity + kBlockKeys - 1) / kBlockKeys, m->c)) return rc;
-    return run_prefill(m, c, ids, n, phase, logits);
+    const int rc = run_prefill(m, c, ids, n, phase, logits);
+    if (rc != YUE2_OK) (void)hipStreamSynchronize(m->stream);  // nothing may still run over the scratch
+    m->scratch.trim();
+    return rc;
 }
 
 extern "C" int32_t yue2_hip_selftest_gemm(const uint16_t* x, const uint16_t* w, float* out, int32_t M, int32_t N,

@@ -668,16 +668,11 @@ int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, b
     const size_t o_x = take(4 * R * H), o_qkv = take(4 * R * qkvw), o_h = take(2 * R * H), o_q = take(2 * R * qw);
     const size_t o_att = take(2 * R * qw), o_act = take(2 * R * I), o_st = take(sizeof(float2) * R * Hq);
     const size_t o_ids = take(sizeof(int32_t) * (size_t)n);
-    struct Scratch {
-        char* p = nullptr;
-        ~Scratch() {
-            if (p) (void)hipFree(p);
-        }
-    } b;
-    if (hipMalloc(&b.p, at) != hipSuccess) {
+    if (m->scratch.ensure(at) != hipSuccess) {
         (void)hipGetLastError();
         return 1;
     }
+    const Scratch& b = m->scratch;
     float *x = reinterpret_cast<float*>(b.p + o_x), *qkv = reinterpret_cast<float*>(b.p + o_qkv);
     uint16_t *h = reinterpret_cast<uint16_t*>(b.p + o_h), *q = reinterpret_cast<uint16_t*>(b.p + o_q);
     uint16_t *att = reinterpret_cast<uint16_t*>(b.p + o_att), *act = reinterpret_cast<uint16_t*>(b.p + o_act);
@@ -713,7 +708,8 @@ int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, b
                 return rc;
             }
     }
-    const hipError_t done = hipStreamSynchronize(s);  // the scratch is freed with nothing running on it
+    const hipError_t done = hipStreamSynchronize(s);  // nothing runs over the scratch any more
+    m->scratch.trim();
     if (e == hipSuccess) e = done;
     return e == hipSuccess ? YUE2_OK : hip_fail(e, "multi-row forward");
 }

@@ -92,7 +92,36 @@ struct NarDev {
 };
 }  // namespace y2
 
+namespace y2 {
+// hipMalloc, tried a second time after the scratch of every model has been
+// given back when the device is out of memory.  Callers hold the library
+// lock and use no scratch yet.
+hipError_t device_malloc_bytes(void** p, size_t bytes);
+template <class T>
+hipError_t device_malloc(T** p, size_t bytes) {
+    return device_malloc_bytes(reinterpret_cast<void**>(p), bytes);
+}
+
+// Device scratch of a model's multi-row calls (prefill, velocity), kept
+// between them: an allocation and its free cost 0.3-5 ms a call, as much as
+// a short prompt's kernels.  At most kScratchKeep bytes stay with an idle
+// model; a larger call's scratch goes back when it ends, all of it with the
+// model or when another allocation needs the memory.  Its user holds the
+// library lock and has finished on the model's stream before it returns.
+struct Scratch {
+    static constexpr size_t kScratchKeep = (size_t)2 << 30;  // a 24000-token prompt of the 3B class: 1.9 GB
+    char* p = nullptr;
+    size_t bytes = 0;
+    hipError_t ensure(size_t want);
+    void release();
+    void trim() {
+        if (bytes > kScratchKeep) release();
+    }
+};
+}  // namespace y2
+
 struct Yue2Model {
+    y2::Scratch scratch;
     Yue2Config c{};
     hipStream_t stream = nullptr;
     void* block = nullptr;

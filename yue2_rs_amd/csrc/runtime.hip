@@ -57,6 +57,37 @@ bool device_ready() {
     return state == 1;
 }
 
+// The live models, whose scratch device_malloc_bytes may take back.
+static std::vector<Yue2Model*> g_models;
+
+hipError_t device_malloc_bytes(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    bool freed = false;
+    for (Yue2Model* m : g_models) {
+        freed = freed || m->scratch.p;
+        m->scratch.release();
+    }
+    if (!freed) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
+hipError_t Scratch::ensure(size_t want) {
+    if (bytes >= want) return hipSuccess;
+    release();
+    const hipError_t e = device_malloc(&p, want);
+    if (e != hipSuccess) p = nullptr;
+    else bytes = want;
+    return e;
+}
+
+void Scratch::release() {
+    if (p) (void)hipFree(p);  // waits for the device
+    p = nullptr;
+    bytes = 0;
+}
+
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Bump allocator over one device allocation.
@@ -118,7 +149,7 @@ int Workspace::ensure(int want_rows, int want_blocks, const Yue2Config& c) {
     const size_t o_st = cv.take<StepState>(1);
     const size_t o_log = cv.take<int32_t>((size_t)log_cap);
     const size_t o_args = cv.take<StepArgs>(1);
-    hipError_t e = hipMalloc(&block, cv.offset);
+    hipError_t e = device_malloc(&block, cv.offset);
     if (e != hipSuccess) {
         block = nullptr;
         return hip_fail(e, "hipMalloc(workspace)");
@@ -150,7 +181,7 @@ int Workspace::ensure(int want_rows, int want_blocks, const Yue2Config& c) {
     // the cleared state) starts at 0 with them
     const FlowLayout fl(c, rows, blk_stride);
     const size_t words = fl.total();
-    e = hipMalloc(&flow_block, words * sizeof(uint64_t));
+    e = device_malloc(&flow_block, words * sizeof(uint64_t));
     if (e != hipSuccess) {
         flow_block = nullptr;
         return hip_fail(e, "hipMalloc(dataflow words)");
@@ -468,6 +499,7 @@ extern "C" Yue2Model* yue2_hip_model_open(const Yue2Config* c, const uint16_t* e
     const int qkvw = (Hq + 2 * Hkv) * D, qw = Hq * D, kw = Hkv * D;
     auto* m = new Yue2Model();
     m->c = *c;
+    g_models.push_back(m);
     Carve cv;
     const size_t o_embed = cv.take<uint16_t>((size_t)V * H);
     const size_t o_head = cv.take<uint16_t>((size_t)V * H);
@@ -491,13 +523,15 @@ extern "C" Yue2Model* yue2_hip_model_open(const Yue2Config* c, const uint16_t* e
     hipError_t e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         hip_fail(e, "hipStreamCreate");
+        g_models.pop_back();
         delete m;
         return nullptr;
     }
-    e = hipMalloc(&m->block, cv.offset);
+    e = device_malloc(&m->block, cv.offset);
     if (e != hipSuccess) {
         hip_fail(e, "hipMalloc(weights)");
         (void)hipStreamDestroy(m->stream);
+        g_models.pop_back();
         delete m;
         return nullptr;
     }
@@ -570,7 +604,7 @@ extern "C" Yue2Model* yue2_hip_model_open(const Yue2Config* c, const uint16_t* e
         up_norm(L.post_norm, src.post_attention_layernorm, H);
     }
     // The layer table in device memory, for the persistent step kernel.
-    if (ok && hipMalloc(&m->layers_dev, sizeof(LayerDev) * m->layers.size()) != hipSuccess) ok = false;
+    if (ok && device_malloc(&m->layers_dev, sizeof(LayerDev) * m->layers.size()) != hipSuccess) ok = false;
     up(m->layers_dev, m->layers.data(), sizeof(LayerDev) * m->layers.size());
     if (ok && (hipDeviceGetAttribute(&m->cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess ||
                m->cus <= 0))
@@ -595,6 +629,8 @@ extern "C" void yue2_hip_model_free(Yue2Model* m) {
     m->decoders.clear();
     m->caches.clear();
     m->ws.release();
+    m->scratch.release();
+    g_models.erase(std::remove(g_models.begin(), g_models.end(), m), g_models.end());
     if (m->layers_dev) (void)hipFree(m->layers_dev);
     if (m->block) (void)hipFree(m->block);
     if (m->nar.block) (void)hipFree(m->nar.block);
@@ -646,7 +682,7 @@ extern "C" Yue2Cache* yue2_hip_cache_new(Yue2Model* m, int32_t capacity) {
     cache->layers = c.num_hidden_layers;
     cache->kv_heads = c.num_key_value_heads;
     cache->head_dim = c.head_dim;
-    hipError_t e = hipMalloc(&cache->kv, elems * sizeof(uint16_t));
+    hipError_t e = device_malloc(&cache->kv, elems * sizeof(uint16_t));
     if (e != hipSuccess) {
         hip_fail(e, "hipMalloc(kv cache)");
         delete cache;

@@ -68,9 +68,9 @@ bool twin_ready() {
     if (!device_ready()) return false;
     TwinState& t = twin();
     if (!t.stream && hipStreamCreateWithFlags(&t.stream, hipStreamNonBlocking) != hipSuccess) return false;
-    if (!t.st && hipMalloc(&t.st, sizeof(StepState)) != hipSuccess) return false;
+    if (!t.st && device_malloc(&t.st, sizeof(StepState)) != hipSuccess) return false;
     if (!t.counters) {
-        if (hipMalloc(&t.counters, 4096 * sizeof(int32_t)) != hipSuccess) return false;
+        if (device_malloc(&t.counters, 4096 * sizeof(int32_t)) != hipSuccess) return false;
         if (hipMemset(t.counters, 0, 4096 * sizeof(int32_t)) != hipSuccess) return false;
     }
     return true;
@@ -82,7 +82,7 @@ void* scratch(size_t bytes) {
     if (t.scratch) (void)hipFree(t.scratch);
     t.scratch = nullptr;
     t.scratch_bytes = 0;
-    if (hipMalloc(&t.scratch, bytes) != hipSuccess) return nullptr;
+    if (device_malloc(&t.scratch, bytes) != hipSuccess) return nullptr;
     t.scratch_bytes = bytes;
     return t.scratch;
 }
@@ -129,7 +129,7 @@ uint16_t* device_weight(const Yue2GpuWeight& w) {
         src = host.data();
     }
     uint16_t* dev = nullptr;
-    if (hipMalloc(&dev, n * sizeof(uint16_t)) != hipSuccess) return nullptr;
+    if (device_malloc(&dev, n * sizeof(uint16_t)) != hipSuccess) return nullptr;
     if (hipMemcpy(dev, src, n * sizeof(uint16_t), hipMemcpyHostToDevice) != hipSuccess) {
         (void)hipFree(dev);
         return nullptr;
@@ -149,7 +149,7 @@ Context* context_entry(const float* k, const float* v, size_t keys, size_t kv, s
         if (e.data) (void)hipFree(e.data);
         e = Context{};
         const size_t capacity = (keys + reserve + 127) & ~(size_t)127;
-        if (hipMalloc(&e.data, 2 * kv * capacity * dim * sizeof(uint16_t)) != hipSuccess) {
+        if (device_malloc(&e.data, 2 * kv * capacity * dim * sizeof(uint16_t)) != hipSuccess) {
             t.contexts.erase({cache, layer});
             return nullptr;
         }
@@ -529,7 +529,7 @@ float* device_weight_f32(const uint8_t* raw, size_t mapping, int dtype, int roun
         host[i] = rounded && dtype != 0 ? rb(v) : v;
     }
     float* dev = nullptr;
-    if (hipMalloc(&dev, host.size() * sizeof(float)) != hipSuccess) return nullptr;
+    if (device_malloc(&dev, host.size() * sizeof(float)) != hipSuccess) return nullptr;
     if (hipMemcpy(dev, host.data(), host.size() * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
         (void)hipFree(dev);
         return nullptr;

@@ -558,7 +558,7 @@ extern "C" Yue2Vae* yue2_hip_vae_open(const char* dir) {
         oi[k] = take(op.ib.size());
     }
     hipError_t e = hipStreamCreateWithFlags(&v->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMalloc(&v->block, std::max<size_t>(total, 256));
+    if (e == hipSuccess) e = device_malloc(&v->block, std::max<size_t>(total, 256));
     if (e != hipSuccess) {
         hip_fail(e, "VAE weights");
         yue2_hip_vae_free(v);
@@ -673,7 +673,7 @@ int vae_decode(Yue2Vae* v, const float* z, int frames, float* out) {
         if (v->acts) (void)hipFree(v->acts);
         v->acts = nullptr;
         v->acts_bytes = 0;
-        if ((e = hipMalloc(&v->acts, 3 * stride)) != hipSuccess) return hip_fail(e, "VAE activations");
+        if ((e = device_malloc(&v->acts, 3 * stride)) != hipSuccess) return hip_fail(e, "VAE activations");
         v->acts_bytes = 3 * stride;
     }
     float* buf[3];
