@@ -1,0 +1,56 @@
+"""The VAE convolutions that run as products of BF16 parts (vae.hip,
+conv_split_kernel): single convolutions against float64 at the sizes where
+the tiles, rings and slots can go wrong, and a whole decoder whose last
+blocks are long enough for the large tile, under the contract of
+test_gpu_vae.py (max |device - f64| <= 4 max |oracle - f64| + 1e-6).
+
+The bound of a single convolution: K products of magnitude below 2.5 * 0.5
+(five sigma each), in at most K / 16 + 6 roundings of a sum below
+0.05 sqrt(K) * 5: K = 910 gives 64 * 7.5 * 2^-24 = 2.9e-5 at worst and
+8 roundings' worth, 4e-6, at random; 1e-5 as test_gpu_vae.py has for FP32."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+import yue2_rs_amd as y2
+
+from test_gpu_vae import _selftest
+from vae_files import conv_case, decode_f64, oracle_ops, synthetic_vae, write_vae_dir
+
+pytestmark = pytest.mark.gpu
+
+# (transpose, cin, cout, kernel, stride, padding, dilation, frames)
+SHAPES = [
+    (False, 16, 17, 7, 1, 3, 1, 1),      # one row, one 16-channel group, a part of one column block
+    (False, 16, 40, 7, 1, 27, 9, 300),   # the widest reach of the 7-tap slots, several row tiles
+    (False, 48, 130, 5, 1, 2, 1, 65),    # a tile and a row; two blocks of padded columns
+    (False, 32, 33, 1, 1, 0, 1, 64),     # one tap, a whole tile
+    (False, 16, 64, 8, 1, 64, 18, 200),  # eight taps, reach 126
+    (False, 128, 20, 2, 1, 32, 65, 129),
+    (True, 32, 64, 20, 10, 5, 1, 40),    # ten phases of two taps
+    (True, 16, 33, 12, 4, 2, 1, 7),      # three taps a phase
+    (False, 16, 32, 7, 1, 3, 1, 49410),  # the large tile, a ragged last one
+    (True, 16, 64, 8, 4, 2, 1, 12300),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_convolution_shapes(gpu, shape):
+    transpose, cin, cout, kernel, stride, padding, dilation, frames = shape
+    x, w, b, want = conv_case(*shape)
+    print(shape, flush=True)
+    got = _selftest(transpose, cin, cout, kernel, stride, padding, dilation, x, w, b, want.shape[0])
+    assert np.abs(got - want).max() <= 1e-5
+
+
+@pytest.mark.parametrize("frames", [1, 37, 1601])
+def test_decode_with_both_tiles(gpu, tmp_path, frames):
+    cfg, t = synthetic_vae(seed=11, channels=32, c_mults=(1, 2), strides=(4, 8))
+    t = {n: a * np.float32(0.5) if n.endswith("weight_g") else a for n, a in t.items()}
+    vae = y2.Vae(write_vae_dir(tmp_path, cfg, t))
+    z = np.random.default_rng(frames).standard_normal((frames, 16)).astype(np.float32)
+    print(f"{frames} frames", flush=True)
+    got, exact = vae.decode(z), decode_f64(cfg, t, z)
+    oracle = oracle_ops(cfg, t).run(z)
+    assert np.abs(got - exact).max() <= 4 * np.abs(oracle - exact).max() + 1e-6
+    vae.close()

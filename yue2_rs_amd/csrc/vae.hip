@@ -20,7 +20,9 @@
 // staged, and a final tanh in the epilogue, so activations never make a
 // round trip through HBM.
 //
-// conv_mfma_kernel: 128 x 128 output tiles, 4 waves of 2 x 2 FP32 MFMA
+// conv_split_kernel: the convolutions of whole 16-channel groups, each FP32
+// product as six products of BF16 parts on the BF16 matrix instructions.
+// conv_mfma_kernel (the other shapes): 128 x 128 output tiles, 4 waves of 2 x 2 FP32 MFMA
 // blocks (v_mfma_f32_32x32x2_f32); per 8-channel chunk the source rows and
 // every tap's weights are staged in LDS (52 KB for 7 taps: two workgroups
 // per CU); step t of a chunk feeds lane half h channel 4h + t, so each lane
@@ -34,8 +36,10 @@
 #include <vector>
 
 #include "../../include/yue2_hip.h"
+#include "dev_mem.h"
 #include "runtime.h"
 #include "vae.h"
+#include "y2_math.h"
 
 using namespace y2;
 
@@ -295,6 +299,278 @@ __global__ __launch_bounds__(256, 2) void conv_mfma_kernel(const ConvPlan p) {
         }
 }
 
+// ---- FP32 convolutions on the BF16 matrix cores ------------------------------
+//
+// Each f32 operand is the exact sum of three BF16 parts (x = x0 + x1 + x2, each
+// the rounding of what is left: 8 + 8 + 8 bits), so x w is the sum of nine
+// BF16 products, of which x1 w2, x2 w1 and x2 w2 are below 2^-26 of it and are
+// left out; six 32x32x16 MFMAs with f32 accumulation replace eight FP32 MFMAs
+// of twice the length each.  Against float64 the six products are three times
+// closer than the FP32 chain (1024 x 1024 outputs: 0.35e-6 against 1.07e-6 at
+// 3584 terms, 0.17e-6 against 0.54e-6 at 896), since sixteen products enter
+// each rounding of the sum.  The parts cover the f32 range; an infinite value
+// gives NaN (SnakeBeta of an infinity already does).
+//
+// Tile: TM = 32 MI WM output rows x TN = 32 NJ WN output channels, one tap of
+// 16 input channels per step.  The weights are split at load and laid out as
+// the MFMA operands of a wave (fragment: 32 channels x 16 inputs of one part,
+// 1 KB, lane order), so a step's slab is one contiguous run that goes straight
+// to LDS, two steps per stage of a ring.  The source rows of XC 16-channel
+// groups are activated and split while the previous chunk is multiplied (their
+// loads were issued a chunk ago) and stored by part and half (8 channels): an
+// operand read is 32 consecutive 16-byte rows, at any tap offset.
+//
+// Bound: BF16 MFMA issue at the clock that random operands leave (a plain BF16
+// GEMM's ~1.1 PFLOP/s, so ~190 TFLOP/s of FP32 products).  Measured on the
+// 1920-ratio shape: 7-tap convolutions 174 TFLOP/s (conv_mfma_kernel 108), the
+// 1-tap ones at 128 channels 5 TB/s; a three-minute song in 512-frame tiles
+// 263 -> 163 ms, 37 frames 6.58 -> 3.31 ms.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) const y2_u32x4 lds_u32x4;
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2w;
+
+// sin(x)^2: x reduced by the nearest multiple of pi (two-part Cody-Waite; the
+// first difference is exact for |x| < 2^22), then the Taylor series of sin to
+// the 13th power on [-pi/2, pi/2] (remainder below 1e-9).  Past 1e5, and for
+// infinities, the library's sinf, decided by the wave.
+__device__ __forceinline__ float sin_squared(float x) {
+    const float n = __builtin_rintf(x * 0.318309886f);
+    float r = __builtin_fmaf(-n, 3.14159274101257324f, x);
+    r = __builtin_fmaf(-n, -8.74227766e-8f, r);
+    const float z = r * r;
+    float q = 1.0f / 6227020800.0f;
+    q = __builtin_fmaf(q, z, -1.0f / 39916800.0f);
+    q = __builtin_fmaf(q, z, 1.0f / 362880.0f);
+    q = __builtin_fmaf(q, z, -1.0f / 5040.0f);
+    q = __builtin_fmaf(q, z, 1.0f / 120.0f);
+    q = __builtin_fmaf(q, z, -1.0f / 6.0f);
+    float t = __builtin_fmaf(q * z, r, r);
+    if (__builtin_amdgcn_ballot_w64(!(__builtin_fabsf(x) <= 1e5f))) t = sinf(x);
+    return t * t;
+}
+
+// The three BF16 parts of two values, as pairs.
+__device__ __forceinline__ void split3(float a, float b, uint32_t* w) {
+    f32x2 v = {a, b};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        w[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2v));
+        if (p < 2) {
+            v[0] -= u2f(w[p] << 16);
+            v[1] -= u2f(w[p] & 0xffff0000u);
+        }
+    }
+}
+
+template <int WM_, int WN_, int MI_, int NJ_>
+struct SplitTile {
+    static constexpr int WM = WM_, WN = WN_, MI = MI_, NJ = NJ_, THREADS = 64 * WM * WN;
+    static constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN;
+    static constexpr int FRAGS = TN / 32 * 3;            // 1 KB fragments of a step's weights
+    static constexpr int LPW = 2 * FRAGS / (WM * WN);    // DMA loads per lane and two-step stage
+    static constexpr int STAGE = 2 * FRAGS * 512;        // BF16 elements of a stage
+    static_assert(2 * FRAGS % (WM * WN) == 0, "whole loads per wave");
+};
+using SplitBig = SplitTile<4, 2, 2, 2>;    // 256 x 128, eight waves
+using SplitSmall = SplitTile<2, 2, 1, 1>;  // 64 x 64, four waves: grids the big tile leaves short
+
+// 16-channel groups per chunk of source rows, stages of the weight ring, and
+// float4 slots per thread for a chunk's rows.
+constexpr int split_xc(int nt) { return nt == 1 ? 2 : 1; }
+constexpr int split_ring(int nt) { return nt == 1 ? 2 : 3; }
+constexpr int split_slots(bool big, int nt) { return big ? (nt == 7 || nt == 2 ? 3 : 4) : nt == 0 ? 3 : 2; }
+template <class T>
+size_t split_lds(int nt, int span) {
+    return (size_t)split_ring(nt) * T::STAGE * 2 + (size_t)2 * split_xc(nt) * 6 * span * 16;
+}
+
+template <int ACT, int NT, class T>
+__global__ __launch_bounds__(T::THREADS, T::THREADS == 512 ? 2 : 1) void conv_split_kernel(const ConvPlan p) {
+    constexpr int XC = split_xc(NT), RING = split_ring(NT), XS = split_slots(T::THREADS == 512, NT);
+    constexpr int GRP = 4 * XC;  // float4 groups of a chunk's row
+    extern __shared__ __align__(16) uint16_t smem[];
+    uint16_t* const ring = smem;
+    uint16_t* const xs = smem + RING * T::STAGE;
+    const int ph = blockIdx.z, m_count = p.m_count[ph];
+    const int m0 = blockIdx.x * T::TM, n0 = blockIdx.y * T::TN;
+    if (m0 >= m_count) return;
+    const int ntaps = NT > 0 ? NT : p.ntaps[ph], span = p.span;
+    const int src_lo = m0 + p.off_min[ph];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, l32 = lane & 31, wm = wave / T::WN, wn = wave % T::WN;
+    const int c16s = p.cin / 16, nchunks = c16s / XC, nblk = p.cout_pad / 32;
+    const int steps = c16s * ntaps, stages = (steps + 1) / 2;
+    // weights: the slab of (tap, 16 channels), all cout: nblk x 3 fragments
+    const uint16_t* wsrc = reinterpret_cast<const uint16_t*>(p.w) + (size_t)(n0 / 32) * 3 * 512 + lane * 8;
+    int next_q = 0, next_c = 0, next_g = 0;  // the next step to request: tap, chunk, group (group outer, tap inner)
+    auto step_base = [&] {
+        const uint16_t* at = wsrc + ((size_t)p.slab[ph][next_q] * c16s + next_c * XC + next_g) * nblk * 3 * 512;
+        if (++next_q == ntaps) {
+            next_q = 0;
+            if (++next_g == XC) {
+                next_g = 0;
+                if (next_c + 1 < nchunks) ++next_c;  // past the end: a slab again, never used
+            }
+        }
+        return at;
+    };
+    auto issue = [&](int buf) {
+        const uint16_t *s0 = step_base(), *s1 = step_base();
+#pragma unroll
+        for (int j = 0; j < T::LPW; ++j) {
+            const int q = wave * T::LPW + j;
+            const uint16_t* at = q >= T::FRAGS ? s1 + (q - T::FRAGS) * 512 : s0 + q * 512;
+            __builtin_amdgcn_global_load_lds((Y2_GLOBAL void*)at, (lds_void*)(ring + buf * T::STAGE + q * 512), 16, 0, 0);
+        }
+    };
+    // source rows: slot s holds item u = tid + THREADS s, row u / GRP, channels 4 (u % GRP) ..
+    f32x4 xr[XS], ar = {}, br = {};
+    const int g4 = tid % GRP;
+    auto load_rows = [&](int ck) {
+        const int ch = ck * 16 * XC + 4 * g4;
+#pragma unroll
+        for (int s = 0; s < XS; ++s) {
+            const int src = min(max(src_lo + (tid + T::THREADS * s) / GRP, 0), p.rows_in - 1);
+            xr[s] = *reinterpret_cast<const f32x4*>(p.x + (size_t)src * p.cin + ch);
+        }
+        if constexpr (ACT == ACT_SNAKE) {
+            ar = *reinterpret_cast<const f32x4*>(p.alpha + ch);
+            br = *reinterpret_cast<const f32x4*>(p.inv_beta + ch);
+        }
+    };
+    auto store_rows = [&](int s, int buf) {
+        const int row = (tid + T::THREADS * s) / GRP, src = src_lo + row;
+        if (row >= span) return;
+        f32x4 v = xr[s];
+        if constexpr (ACT == ACT_SNAKE) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = v[e] + br[e] * sin_squared(v[e] * ar[e]);
+        } else if constexpr (ACT == ACT_ELU) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = v[e] < 0.0f ? expf(v[e]) - 1.0f : v[e];
+        }
+        const bool in = src >= 0 && src < p.rows_in;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = in ? v[e] : 0.0f;
+        uint32_t lo[3], hi[3];
+        split3(v[0], v[1], lo);
+        split3(v[2], v[3], hi);
+#pragma unroll
+        for (int part = 0; part < 3; ++part) {
+            const int unit = (((buf * XC + (g4 >> 2)) * 3 + part) * 2 + ((g4 >> 1) & 1)) * span + row;
+            *(lds_u32x2w*)(xs + unit * 8 + (g4 & 1) * 4) = u32x2{lo[part], hi[part]};
+        }
+    };
+    f32x16 acc[T::MI][T::NJ];
+#pragma unroll
+    for (int i = 0; i < T::MI; ++i)
+#pragma unroll
+        for (int j = 0; j < T::NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    int t = 0, slot = 0;  // the step, and its stage's place in the ring
+    auto multiply = [&](int xbuf, int g, int off) {
+        if (t > 0 && !(t & 1)) {
+            // stage t / 2 has landed (later loads may be in flight) and every
+            // wave has read the stage before, whose buffer takes the next one
+            const int s = t >> 1;
+            if (RING > 2 && s - 2 + RING < stages)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((RING - 2) * T::LPW) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            asm volatile("s_barrier" ::: "memory");
+            if (s - 1 + RING < stages) issue(slot);
+            slot = slot + 1 == RING ? 0 : slot + 1;
+        }
+        const uint16_t* wb = ring + slot * T::STAGE + ((t & 1) * T::FRAGS + wn * T::NJ * 3) * 512 + lane * 8;
+        const uint16_t* xb = xs + (((xbuf * XC + g) * 6 + h) * span + wm * T::MI * 32 + l32 + off) * 8;
+        y2_u32x4 a[3][T::MI], b[3][T::NJ];
+#pragma unroll
+        for (int part = 2; part >= 0; --part) {
+#pragma unroll
+            for (int i = 0; i < T::MI; ++i) a[part][i] = *(lds_u32x4*)(xb + (part * 2 * span + i * 32) * 8);
+#pragma unroll
+            for (int j = 0; j < T::NJ; ++j) b[part][j] = *(lds_u32x4*)(wb + (j * 3 + part) * 512);
+        }
+        auto product = [&](int pa, int pb) {
+#pragma unroll
+            for (int i = 0; i < T::MI; ++i)
+#pragma unroll
+                for (int j = 0; j < T::NJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[pa][i]),
+                                                                        __builtin_bit_cast(bf16x8, b[pb][j]),
+                                                                        acc[i][j], 0, 0, 0);
+        };
+        product(2, 0);
+        product(0, 2);
+        product(1, 1);
+        product(1, 0);
+        product(0, 1);
+        product(0, 0);
+        ++t;
+    };
+    load_rows(0);
+    for (int s = 0; s < min(stages, RING); ++s) issue(s);
+#pragma unroll
+    for (int s = 0; s < XS; ++s) store_rows(s, 0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    for (int ck = 0; ck < nchunks; ++ck) {
+        const bool more = ck + 1 < nchunks;
+        if (more) load_rows(ck + 1);
+        if constexpr (NT > 0) {
+            constexpr int SPC = NT * XC;
+#pragma unroll
+            for (int k = 0; k < SPC; ++k) {
+                multiply(ck & 1, k / NT, p.off[ph][k % NT] - p.off_min[ph]);
+                // the next chunk's slots over the last steps
+                if (more)
+#pragma unroll
+                    for (int s = 0; s < XS; ++s)
+                        if (XS >= SPC ? s * SPC / XS == k : k == SPC - XS + s) store_rows(s, (ck + 1) & 1);
+            }
+        } else {
+            for (int q = 0; q < ntaps; ++q) multiply(ck & 1, 0, p.off[ph][q] - p.off_min[ph]);
+            if (more)
+#pragma unroll
+                for (int s = 0; s < XS; ++s) store_rows(s, (ck + 1) & 1);
+        }
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            asm volatile("s_barrier" ::: "memory");  // chunk ck + 1 is staged, chunk ck read by every wave
+        }
+    }
+    const int ostride = p.ostride, o0 = p.o0[ph], cout = p.cout;
+#pragma unroll
+    for (int i = 0; i < T::MI; ++i)
+#pragma unroll
+        for (int j = 0; j < T::NJ; ++j) {
+            const int o = n0 + (wn * T::NJ + j) * 32 + l32, oc = min(o, cout - 1);
+            const int mb = m0 + (wm * T::MI + i) * 32 + 4 * h;
+            const float bias = p.b ? p.b[oc] : 0.0f;
+            float rv[16];
+            if (p.res) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    rv[r] = p.res[(size_t)(o0 + ostride * min(mb + 8 * (r >> 2) + (r & 3), m_count - 1)) * cout + oc];
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = mb + 8 * (r >> 2) + (r & 3);
+                if (m < m_count && o < cout) {
+                    float v = acc[i][j][r] + bias;  // Conv::apply: the product, then the bias
+                    if (p.res) v = v + rv[r];       // Op::Residual: h + x
+                    if (p.tanh_out) v = tanhf(v);
+                    p.y[(size_t)(o0 + ostride * m) * cout + o] = v;
+                }
+            }
+        }
+}
+
 // Weight slabs [k][cin_pad][CO]; one output row per thread.
 template <int CO, int ACT>
 __global__ __launch_bounds__(256) void conv_narrow_kernel(const ConvPlan p) {
@@ -363,8 +639,13 @@ int conv_length(const VaeOpHost& op, int n) {
 // The device form of one convolution: which kernel, its channel chunk and
 // padded widths.
 struct ConvShape {
-    bool mfma = false;
+    bool mfma = false, split = false;  // split: mfma on the BF16 parts
     int chunk = kChunk, cin_pad = 0, cout_pad = 0;
+    // floats of the weight slabs (three BF16 parts are 1.5 floats)
+    size_t weights(int kernel) const {
+        const size_t n = (size_t)kernel * cin_pad * cout_pad;
+        return split ? (n * 3 + 1) / 2 : n;
+    }
 };
 
 // Source rows a 128-row output tile reads: at most 160 (32-channel chunks)
@@ -374,9 +655,28 @@ int mfma_span(const VaeOpHost& op) {
     return (kMmaTile - 1) * op.stride + op.dilation * (op.kernel - 1) + 1;
 }
 
+// Whether a convolution runs on the BF16 parts: whole 16-channel groups, unit
+// source stride, at most kMaxTaps taps in every phase and rows within the
+// slots of both tiles (64 + 128 rows for the small one).  The others (odd
+// channel counts, strided convolutions, phases without a tap) stay on the
+// FP32 instructions.
+bool split_shape(const VaeOpHost& op) {
+    if (op.cout <= 16 || op.cin % 16) return false;
+    if (op.kind == VAE_CONVT)
+        return op.dilation == 1 && op.stride <= kMaxPhases && op.kernel % op.stride == 0 && op.kernel / op.stride <= kMaxTaps;
+    return op.stride == 1 && op.kernel <= kMaxTaps && op.dilation * (op.kernel - 1) <= (op.kernel == 7 ? 54 : 128);
+}
+
 ConvShape conv_shape(const VaeOpHost& op) {
     ConvShape c;
     c.mfma = op.cout > 16;
+    c.split = split_shape(op);
+    if (c.split) {
+        c.chunk = 16;
+        c.cin_pad = op.cin;
+        c.cout_pad = (op.cout + kMmaTile - 1) / kMmaTile * kMmaTile;
+        return c;
+    }
     const int taps = op.kind == VAE_CONVT ? (op.kernel + op.stride - 1) / op.stride : op.kernel;
     const bool uniform = op.kind == VAE_CONV || op.kernel % op.stride == 0;  // every phase has `taps` taps
     c.chunk = !c.mfma ? kChunk : taps <= 2 && uniform && op.cin % 4 == 0 && mfma_span(op) <= 160 ? 32 : 8;
@@ -389,8 +689,26 @@ ConvShape conv_shape(const VaeOpHost& op) {
 // Tap slabs in the kernel's layout from the checkpoint layout ([out, in, k]
 // or, for a transposed convolution, [in, out, k]); zero padding.
 std::vector<float> conv_slabs(const VaeOpHost& op, const ConvShape& c) {
-    std::vector<float> t((size_t)op.kernel * c.cin_pad * c.cout_pad, 0.0f);
+    std::vector<float> t(c.weights(op.kernel), 0.0f);
     const int nchunks = c.cin_pad / c.chunk;
+    if (c.split) {
+        // [tap][16 inputs][32 outputs][part][lane: output l % 32, inputs 8 (l / 32) ..][8]
+        uint16_t* d = reinterpret_cast<uint16_t*>(t.data());
+        for (int o = 0; o < op.cout; ++o)
+            for (int i = 0; i < op.cin; ++i)
+                for (int j = 0; j < op.kernel; ++j) {
+                    float v = op.w[op.kind == VAE_CONVT ? ((size_t)i * op.cout + o) * op.kernel + j
+                                                        : ((size_t)o * op.cin + i) * op.kernel + j];
+                    const size_t frag = (((size_t)j * nchunks + i / 16) * (c.cout_pad / 32) + o / 32) * 3;
+                    const size_t in = (size_t)((i % 16 / 8) * 32 + o % 32) * 8 + i % 8;
+                    for (int part = 0; part < 3; ++part) {
+                        const float r = rb(v);
+                        d[(frag + part) * 512 + in] = bf16_bits(r);
+                        v -= r;
+                    }
+                }
+        return t;
+    }
     for (int o = 0; o < op.cout; ++o)
         for (int i = 0; i < op.cin; ++i)
             for (int j = 0; j < op.kernel; ++j) {
@@ -410,6 +728,46 @@ hipError_t launch(K kernel, dim3 grid, size_t lds, hipStream_t s, const ConvPlan
                               (int)lds);
     kernel<<<grid, 256, lds, s>>>(p);
     return hipGetLastError();
+}
+
+template <int ACT, int NT, class T>
+hipError_t launch_split(const ConvPlan& p, int mrows, int phases, hipStream_t s) {
+    const size_t lds = split_lds<T>(NT, p.span);
+    if (lds > kMaxLds || p.span * 4 * split_xc(NT) > T::THREADS * split_slots(T::THREADS == 512, NT))
+        return hipErrorInvalidValue;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_split_kernel<ACT, NT, T>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    conv_split_kernel<ACT, NT, T>
+        <<<dim3((mrows + T::TM - 1) / T::TM, (p.cout_pad + T::TN - 1) / T::TN, phases), T::THREADS, lds, s>>>(p);
+    return hipGetLastError();
+}
+
+// A split convolution: p filled but for the span, which the tile decides.
+hipError_t run_split(ConvPlan& p, int act, int phases, hipStream_t s) {
+    int rows = 0, reach = 0;
+    for (int ph = 0; ph < phases; ++ph) {
+        rows = std::max(rows, p.m_count[ph]);
+        for (int q = 0; q < p.ntaps[ph]; ++q) reach = std::max(reach, p.off[ph][q] - p.off_min[ph]);
+    }
+    const long tiles = (long)((rows + SplitBig::TM - 1) / SplitBig::TM) * (p.cout_pad / SplitBig::TN) * phases;
+    // half the CUs with a big tile each beat 64 x 64 tiles (song 163 ms;
+    // 166 from 192 tiles on, 168 from 300), a quarter do not (37 frames 3.62
+    // against 3.34 ms)
+    const bool big = tiles >= 128;
+    p.span = (big ? SplitBig::TM : SplitSmall::TM) + reach;
+#define Y2_SPLIT(ACT, NT)                                                     \
+    return big ? launch_split<ACT, NT, SplitBig>(p, rows, phases, s)          \
+               : launch_split<ACT, NT, SplitSmall>(p, rows, phases, s);
+    if (act == ACT_SNAKE) {
+        if (p.ltaps == 7 && reach <= 64) { Y2_SPLIT(ACT_SNAKE, 7) }
+        if (p.ltaps == 2 && reach <= 64) { Y2_SPLIT(ACT_SNAKE, 2) }  // (the small tile's slots)
+        if (p.ltaps == 1 && p.cin % 32 == 0) { Y2_SPLIT(ACT_SNAKE, 1) }
+        Y2_SPLIT(ACT_SNAKE, 0)
+    }
+    if (act == ACT_ELU) { Y2_SPLIT(ACT_ELU, 0) }
+    Y2_SPLIT(ACT_NONE, 0)
+#undef Y2_SPLIT
 }
 
 // One convolution (plain or transposed) of x [n, cin] into y [length, cout]:
@@ -462,6 +820,7 @@ hipError_t run_conv(hipStream_t s, const VaeOpHost& op, const ConvShape& c, cons
         mtiles = std::max(mtiles, (p.m_count[ph] + tile - 1) / tile);
     }
     if (mtiles == 0) return hipSuccess;
+    if (c.split) return run_split(p, act, phases, s);
     const size_t pitch = c.chunk + 4;
     const size_t lds = c.mfma ? sizeof(float) * ((size_t)p.ltaps * kMmaTile * pitch + (size_t)p.span * pitch)
                               : sizeof(float) * ((size_t)p.ltaps * kChunk * c.cout_pad + (size_t)p.span * kNarrowPad);
@@ -552,7 +911,7 @@ extern "C" Yue2Vae* yue2_hip_vae_open(const char* dir) {
     for (size_t k = 0; k < nops; ++k) {
         const VaeOpHost& op = v->host.ops[k];
         if (op.kind == VAE_CONV || op.kind == VAE_CONVT) v->shape[k] = conv_shape(op);
-        ow[k] = take((size_t)op.kernel * v->shape[k].cin_pad * v->shape[k].cout_pad);
+        ow[k] = take(v->shape[k].weights(op.kernel));
         ob[k] = take(op.b.size());
         oa[k] = take(op.a.size());
         oi[k] = take(op.ib.size());
