@@ -75,15 +75,26 @@ def test_prompt_equals_token_steps(shape, n):
     _check(shape[2], 0, n, seed=n)
 
 
-@pytest.mark.parametrize("context,n", [(1, 4), (63, 5), (100, 37), (500, 130)])
+@pytest.mark.parametrize("context,n", [(1, 5), (63, 5), (100, 37), (500, 130)])
 def test_append_equals_token_steps(shape, context, n):
     _check(shape[2], context, n, seed=context + n)
 
 
-@pytest.mark.parametrize("context,n", [(16200, 121), (16255, 130), (16256, 129), (16400, 130)])
+@pytest.mark.parametrize("context,n", [(16290, 32), (16255, 130), (16256, 129), (16400, 35)])
 def test_long_append_equals_token_steps(shape, context, n):
     if shape[0] in ("d64", "d128"):
         _check(shape[2], context, n, seed=context + n)
+
+
+# from 256 workgroups of 128 rows on, past 256 blocks: the attention kernels of
+# long contexts, their last workgroup with seven rows; and as many without a
+# context
+@pytest.mark.parametrize("context,n", [(0, 1), (13100, 7)])
+def test_many_rows_equal_token_steps(shape, context, n):
+    name, _, gm = shape
+    if name in ("d64", "d128"):
+        rows = 128 * (255 // gm.config.num_attention_heads + 1)
+        _check(gm, context, rows - 128 + n, seed=n)
 
 
 def test_prompt_equals_oracle(gpu, oracle_threads):

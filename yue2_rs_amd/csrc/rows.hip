@@ -294,9 +294,16 @@ hipError_t launch_dot_gemm(hipStream_t s, int epi, const GemmArgs& g) {
 // recomputed each time (an f32 score matrix costs as much to write and read
 // back, and grows with the square of the context).
 //
-// One workgroup per (query head, 128 query rows): eight waves of 16 queries,
-// 64-key blocks of K (and V transposed) staged in LDS for all of them.  The
-// scores are computed transposed, S^T = K Q^T with 16x16x4 MFMAs: lane l has
+// Two forms.  Up to kLongKeys keys, and for few rows, the four waves of a
+// workgroup share 16 queries (share_*_kernel); for many rows of a longer
+// context a workgroup takes 128 rows, a wave 16 of them alone (rows_*_kernel).
+// Prompts of two layers through either, ms: 3B class 9.95 against 10.29 at
+// 2048 tokens, 37.3 / 38.4 at 6000, 98.4 / 95.7 at 12000, 244 / 215 at 20000
+// (the block sums of 313 blocks leave the shared statistics one workgroup per
+// CU); a 1B class 6.64 / 6.75, 24.8 / 25.6, 68.5 / 70.2, 108 / 112 at 16000.
+// 517 tokens of the YuE2 shape, per layer: 77 us against 236.
+//
+// The scores are computed transposed, S^T = K Q^T with 16x16x4 MFMAs: lane l has
 // query l % 16 and, of the block, keys 16 kt + 4 (l / 16) + r.  A score's
 // D / 8 chunk chains (two MFMAs each, from +0) are added as they end, in
 // bit-reversed order, which is the butterfly over distances D/16 .. 1.
@@ -307,18 +314,18 @@ hipError_t launch_dot_gemm(hipStream_t s, int epi, const GemmArgs& g) {
 // are eight streams, 4 (j & 1) + r: two passes with the other lanes' p zero
 // (an fma of zeros leaves a chain that starts at +0 as it is).
 //
-// Bound: the FP32 MFMAs (4 x 4096 cycles per wave and 64-key block), with the
-// f64 exponentials and the divisions (~3000 cycles) beside them on the vector
-// ALU of other waves.
-constexpr int kRowsQ = 128, kRowsThreads = 512, kLongKeys = 255 * kBlockKeys;
+// Bound: the FP32 MFMAs (4 x 4096 cycles per 16 queries and 64-key block) and
+// the vector ALU beside them (unpacking, the trees, the f64 exponentials and
+// the divisions: ~6000 cycles), which share their issue time.
+constexpr int kRowsQ = 128, kRowsThreads = 512, kRowsWaves = 8, kLongKeys = 255 * kBlockKeys;
 
 template <int D>
 __device__ __forceinline__ int key_swz(int key) { return D == 128 ? key & 15 : (key >> 1) & 7; }
 
 // Requests the K rows of block t (keys past last: the last one) into LDS.
-template <int D>
+template <int D, int NW>
 __device__ __forceinline__ void stage_keys(const uint16_t* K, int t, int last, uint16_t* dst) {
-    constexpr int U = D / 8, LPW = kBlockKeys * U / kRowsThreads;
+    constexpr int U = D / 8, LPW = kBlockKeys * U / (64 * NW);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
     for (int j = 0; j < LPW; ++j) {
@@ -338,49 +345,115 @@ __device__ __forceinline__ void load_query(const uint16_t* q, bool in, float (&q
         for (int s = 0; s < 2; ++s) qf[c][s] = in ? bf16(gbl(q)[8 * c + 4 * s + j]) : 0.0f;
 }
 
-// The DOTs of the block's 64 keys with the wave's queries.
+// The DOTs of 32 staged keys (two 16-key tiles) with the wave's queries.
 template <int D>
-__device__ __forceinline__ void block_scores(const uint16_t* ks, const float (&qf)[D / 8][2], f32x4 (&s)[4]) {
+__device__ __forceinline__ void half_scores(const uint16_t* ks, const float (&qf)[D / 8][2], f32x4 (&s)[2]) {
     constexpr int NC = D / 8, LV = D == 128 ? 4 : 3;
     const int lane = threadIdx.x & 63, j = lane >> 4;
     const uint32_t sel = (j & 1) ? kSelHi : kSelLo;
     typedef __attribute__((address_space(3))) const uint32_t lds_u32;
     const int swz = key_swz<D>(lane & 15);
     const uint16_t* row = ks + (lane & 15) * D + (j >> 1) * 2;
+    f32x4 st[LV][2];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ci = 0; ci < NC; ++ci) {
+        int c = 0;  // bit-reversed ci
+#pragma unroll
+        for (int b = 0; b < LV; ++b) c |= ((ci >> b) & 1) << (LV - 1 - b);
+        const uint16_t* at = row + ((c ^ swz) << 3);
+        f32x4 acc[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const uint32_t w0 = *(lds_u32*)(at + u * 16 * D), w1 = *(lds_u32*)(at + u * 16 * D + 4);
+            const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            acc[u] = mfma_f32_16(bf16_sel(w0, sel), qf[c][0], zero);
+            acc[u] = mfma_f32_16(bf16_sel(w1, sel), qf[c][1], acc[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            bool done = false;
+#pragma unroll
+            for (int v = 0; v < LV; ++v) {
+                if (done) continue;
+                if ((ci >> v) & 1) acc[u] = st[v][u] + acc[u];
+                else {
+                    st[v][u] = acc[u];
+                    done = true;
+                }
+            }
+            if (ci == NC - 1) s[u] = acc[u];
+        }
+    }
+}
+
+// The same of 16 staged keys (one tile).
+template <int D>
+__device__ __forceinline__ void tile_scores(const uint16_t* ks, const float (&qf)[D / 8][2], f32x4& s) {
+    constexpr int NC = D / 8;
+    const int lane = threadIdx.x & 63, j = lane >> 4;
+    const uint32_t sel = (j & 1) ? kSelHi : kSelLo;
+    typedef __attribute__((address_space(3))) const uint32_t lds_u32;
+    const uint16_t* row = ks + (lane & 15) * D + (j >> 1) * 2;
+    f32x4 p[NC];  // the chunk chains, then the butterfly over distances NC / 2 .. 1
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const uint16_t* at = row + ((c ^ key_swz<D>(lane & 15)) << 3);
+        const uint32_t w0 = *(lds_u32*)(at), w1 = *(lds_u32*)(at + 4);
+        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        p[c] = mfma_f32_16(bf16_sel(w0, sel), qf[c][0], zero);
+        p[c] = mfma_f32_16(bf16_sel(w1, sel), qf[c][1], p[c]);
+    }
+#pragma unroll
+    for (int d = NC / 2; d >= 1; d >>= 1)
+#pragma unroll
+        for (int c = 0; c < d; ++c) p[c] = p[c] + p[c + d];
+    s = p[0];
+}
+
+// One block's PV for 16 dims (vrow: this lane's row of the transposed V tile):
+// the streams' fma chains over the block's keys, then their butterfly.
+template <int D>
+__device__ __forceinline__ f32x4 pv_tile(const uint16_t* vrow, const f32x4 (&p)[4]) {
+    const int lane = threadIdx.x & 63, j = lane >> 4, swz = (lane & 15) >> 1;
+    const y2_u32x4 w0 = *(lds_u32x4*)(vrow + ((2 * j) ^ swz) * 8);
+    const y2_u32x4 w1 = *(lds_u32x4*)(vrow + ((2 * j + 1) ^ swz) * 8);
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 acc[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float fv[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            const uint32_t w = (kt < 2 ? w0 : w1)[(kt & 1) * 2 + (e >> 1)];
+            fv[kt] = e & 1 ? bf16_hi(w) : bf16_lo(w);
+        }
+        if constexpr (D == 128) {
+            acc[e] = zero;
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) acc[e] = mfma_f32_16(fv[kt], p[kt][e], acc[e]);
+        } else {
+            f32x4 a0 = zero, a1 = zero;  // streams e and 4 + e
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+                a0 = mfma_f32_16(fv[kt], j & 1 ? 0.0f : p[kt][e], a0);
+                a1 = mfma_f32_16(fv[kt], j & 1 ? p[kt][e] : 0.0f, a1);
+            }
+            acc[e] = a0 + a1;
+        }
+    }
+    return (acc[0] + acc[2]) + (acc[1] + acc[3]);
+}
+
+// The DOTs of a block's 64 keys.
+template <int D>
+__device__ __forceinline__ void block_scores(const uint16_t* ks, const float (&qf)[D / 8][2], f32x4 (&s)[4]) {
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-        f32x4 st[LV][2];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ci = 0; ci < NC; ++ci) {
-            int c = 0;  // bit-reversed ci
-#pragma unroll
-            for (int b = 0; b < LV; ++b) c |= ((ci >> b) & 1) << (LV - 1 - b);
-            const uint16_t* at = row + ((c ^ swz) << 3);
-            f32x4 acc[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int kt = 2 * half + u;
-                const uint32_t w0 = *(lds_u32*)(at + kt * 16 * D), w1 = *(lds_u32*)(at + kt * 16 * D + 4);
-                const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc[u] = mfma_f32_16(bf16_sel(w0, sel), qf[c][0], zero);
-                acc[u] = mfma_f32_16(bf16_sel(w1, sel), qf[c][1], acc[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                bool done = false;
-#pragma unroll
-                for (int v = 0; v < LV; ++v) {
-                    if (done) continue;
-                    if ((ci >> v) & 1) acc[u] = st[v][u] + acc[u];
-                    else {
-                        st[v][u] = acc[u];
-                        done = true;
-                    }
-                }
-                if (ci == NC - 1) s[2 * half + u] = acc[u];
-            }
-        }
+        f32x4 t[2];
+        half_scores<D>(ks + half * 32 * D, qf, t);
+        s[2 * half] = t[0];
+        s[2 * half + 1] = t[1];
     }
 }
 
@@ -430,10 +503,10 @@ __device__ __forceinline__ RowsQuery rows_query(const FlashArgs& f) {
     return r;
 }
 
-// LONG: some row attends more than kLongKeys keys (256 blocks), whose blocks
-// are then added in pairs (super-blocks of 2): blocks are taken two at a
-// time, a last odd one with an empty partner.
-template <int D, bool LONG>
+// Contexts past kLongKeys (256 blocks), whose blocks are added in pairs
+// (super-blocks of 2): blocks are taken two at a time, a last odd one with an
+// empty partner.  A row of fewer blocks beside a longer one adds them singly.
+template <int D>
 __global__ __launch_bounds__(kRowsThreads, 2) void rows_stats_kernel(const FlashArgs f, float2* stats) {
     __shared__ __align__(16) uint16_t ks[2][kBlockKeys * D];
     const RowsQuery r = rows_query(f);
@@ -441,16 +514,16 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_stats_kernel(const Flash
     const uint16_t* K = f.kv_base + (((size_t)f.layer * 2) * f.kv_heads + r.g) * (size_t)f.cap * D;
     float qf[D / 8][2];
     load_query<D>(f.q + ((size_t)min(r.qrow, f.rows - 1) * f.heads + r.h) * D, r.in, qf);
-    const int tiles = LONG ? (r.tiles + 1) & ~1 : r.tiles;
-    const bool two = LONG && (r.qpos + kBlockKeys) / kBlockKeys >= 256;
+    const int tiles = (r.tiles + 1) & ~1;
+    const bool two = (r.qpos + kBlockKeys) / kBlockKeys >= 256;
     float m = -__builtin_huge_valf(), total = 0.0f, part = 0.0f;
-    stage_keys<D>(K, 0, last, ks[0]);
+    stage_keys<D, kRowsWaves>(K, 0, last, ks[0]);
     for (int it = 0; it < 2 * tiles; ++it) {
         const bool sums = it >= tiles;
         const int t = sums ? it - tiles : it, kb = t * kBlockKeys;
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         asm volatile("s_barrier" ::: "memory");  // block t is staged, block t - 1 read by every wave
-        if (it + 1 < 2 * tiles) stage_keys<D>(K, it + 1 < tiles ? it + 1 : it + 1 - tiles, last, ks[(it + 1) & 1]);
+        if (it + 1 < 2 * tiles) stage_keys<D, kRowsWaves>(K, it + 1 < tiles ? it + 1 : it + 1 - tiles, last, ks[(it + 1) & 1]);
         if (it == tiles) m = xor_max<32, 16>(m) * f.scale;  // the scaled maximum (rounding is monotonic)
         float u = 0.0f;
         if (kb <= r.wave_last) {
@@ -482,9 +555,7 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_stats_kernel(const Flash
             u = (v[0] + v[2]) + (v[1] + v[3]);
         }
         if (!sums) continue;
-        if constexpr (!LONG) {
-            total = t == 0 ? u : total + u;
-        } else if (t & 1) {
+        if (t & 1) {
             const float pair = part + u;
             total = t == 1 ? pair : two ? total + pair : (total + part) + u;
         } else {
@@ -494,10 +565,10 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_stats_kernel(const Flash
     if (r.in && j == 0) stats[(size_t)r.qrow * f.heads + r.h] = make_float2(m, total);
 }
 
-template <int D, bool LONG>
+template <int D>
 __global__ __launch_bounds__(kRowsThreads, 2) void rows_pv_kernel(const FlashArgs f, const float2* stats) {
     constexpr int VU = kBlockKeys / 2 * (D / 8);  // V units: a key pair x 8 dims
-    static_assert(VU <= kRowsThreads, "one V unit per thread");
+    constexpr int VS = (VU + kRowsThreads - 1) / kRowsThreads;  // units per thread
     __shared__ __align__(16) uint16_t ks[2][kBlockKeys * D];
     // V transposed: row = dim, key 16 kt + 4 j + r at 16 j + 4 kt + r (a
     // lane's keys are 16 consecutive halfwords), 16-byte units swizzled
@@ -509,27 +580,33 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_pv_kernel(const FlashArg
     float qf[D / 8][2];
     load_query<D>(f.q + ((size_t)min(r.qrow, f.rows - 1) * f.heads + r.h) * D, r.in, qf);
     const float2 mt = r.in ? stats[(size_t)r.qrow * f.heads + r.h] : make_float2(0.0f, 1.0f);
-    const int tiles = LONG ? (r.tiles + 1) & ~1 : r.tiles;
-    const bool two = LONG && (r.qpos + kBlockKeys) / kBlockKeys >= 256;
-    f32x4 o[D / 16], pend[LONG ? D / 16 : 1];
+    const int tiles = (r.tiles + 1) & ~1;
+    const bool two = (r.qpos + kBlockKeys) / kBlockKeys >= 256;
+    f32x4 o[D / 16], pend[D / 16];
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int vp = tid % (kBlockKeys / 2), vd = tid / (kBlockKeys / 2) * 8;  // this thread's V unit
-    uint4 va, vb;
+    // this thread's V units
+    uint4 va[VS], vb[VS];
     auto load_values = [&](int t) {
-        const int k = t * kBlockKeys + 2 * vp;
-        if (tid < VU) {
-            va = ldg4(V + (size_t)min(k, last) * D + vd);
-            vb = ldg4(V + (size_t)min(k + 1, last) * D + vd);
+#pragma unroll
+        for (int i = 0; i < VS; ++i) {
+            const int u = tid + kRowsThreads * i, k = t * kBlockKeys + 2 * (u % (kBlockKeys / 2)), vd = u / (kBlockKeys / 2) * 8;
+            if (u < VU) {
+                va[i] = ldg4(V + (size_t)min(k, last) * D + vd);
+                vb[i] = ldg4(V + (size_t)min(k + 1, last) * D + vd);
+            }
         }
     };
-    stage_keys<D>(K, 0, last, ks[0]);
+    stage_keys<D, kRowsWaves>(K, 0, last, ks[0]);
     load_values(0);
     for (int t = 0; t < tiles; ++t) {
         const int kb = t * kBlockKeys, buf = t & 1;
-        if (tid < VU) {
-            const int k = 2 * vp, unit = 2 * ((k >> 2) & 3) + (k >> 5), in = ((k >> 4) & 1) * 4 + (k & 3);
-            const uint32_t a[4] = {va.x, va.y, va.z, va.w}, b[4] = {vb.x, vb.y, vb.z, vb.w};
+#pragma unroll
+        for (int i = 0; i < VS; ++i) {
+            const int u = tid + kRowsThreads * i, vd = u / (kBlockKeys / 2) * 8;
+            if (u >= VU) continue;
+            const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), in = ((k >> 4) & 1) * 4 + (k & 3);
+            const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, b[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int d = vd + e;
@@ -541,11 +618,10 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_pv_kernel(const FlashArg
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         asm volatile("s_barrier" ::: "memory");  // block t is staged, block t - 1 read by every wave
         if (t + 1 < tiles) {
-            stage_keys<D>(K, t + 1, last, ks[buf ^ 1]);
+            stage_keys<D, kRowsWaves>(K, t + 1, last, ks[buf ^ 1]);
             load_values(t + 1);
         }
         const bool live = kb <= r.wave_last;
-        if (!LONG && !live) continue;
         f32x4 p[4];
         if (live) {
             block_scores<D>(ks[buf], qf, p);
@@ -563,41 +639,9 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_pv_kernel(const FlashArg
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) {
             f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (live) {
-                const uint16_t* vrow = &vt[buf][(dt * 16 + (lane & 15)) * kBlockKeys];
-                const int swz = (lane & 15) >> 1;
-                const y2_u32x4 w0 = *(lds_u32x4*)(vrow + ((2 * j) ^ swz) * 8);
-                const y2_u32x4 w1 = *(lds_u32x4*)(vrow + ((2 * j + 1) ^ swz) * 8);
-                f32x4 acc[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float fv[4];
-#pragma unroll
-                    for (int kt = 0; kt < 4; ++kt) {
-                        const uint32_t w = (kt < 2 ? w0 : w1)[(kt & 1) * 2 + (e >> 1)];
-                        fv[kt] = e & 1 ? bf16_hi(w) : bf16_lo(w);
-                    }
-                    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (D == 128) {
-                        acc[e] = zero;
-#pragma unroll
-                        for (int kt = 0; kt < 4; ++kt) acc[e] = mfma_f32_16(fv[kt], p[kt][e], acc[e]);
-                    } else {
-                        f32x4 a0 = zero, a1 = zero;  // streams e and 4 + e
-#pragma unroll
-                        for (int kt = 0; kt < 4; ++kt) {
-                            a0 = mfma_f32_16(fv[kt], j & 1 ? 0.0f : p[kt][e], a0);
-                            a1 = mfma_f32_16(fv[kt], j & 1 ? p[kt][e] : 0.0f, a1);
-                        }
-                        acc[e] = a0 + a1;
-                    }
-                }
-                v = (acc[0] + acc[2]) + (acc[1] + acc[3]);
-            }
+            if (live) v = pv_tile<D>(&vt[buf][(dt * 16 + (lane & 15)) * kBlockKeys], p);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (!LONG) {
-                o[dt] = t == 0 ? v : o[dt] + v;
-            } else if (t & 1) {
+            if (t & 1) {
                 const f32x4 pair = pend[dt] + v, a = o[dt] + pair, b = (o[dt] + pend[dt]) + v;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[dt][e] = t == 1 ? pair[e] : two ? a[e] : b[e];
@@ -617,17 +661,226 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_pv_kernel(const FlashArg
     }
 }
 
-hipError_t launch_rows_attention(hipStream_t s, const FlashArgs& f, float2* stats, int head_dim) {
-    const dim3 grid(f.heads, (f.rows + kRowsQ - 1) / kRowsQ);
-    const bool lng = f.p0 + f.rows > kLongKeys;
-    auto run = [&](auto stat, auto pv) {
-        stat<<<grid, kRowsThreads, 0, s>>>(f, stats);
-        pv<<<grid, kRowsThreads, 0, s>>>(f, stats);
+// The four waves of a workgroup share 16 queries.  A wave of the kernels above
+// walks every key block of its queries alone, ~6 us a block in each kernel.
+// Here the statistics' blocks are dealt to the waves (maxima and block sums are exchanged through LDS, the
+// sums added in block order at the end), and of each PV block a wave computes
+// the p of 16 keys and, from everyone's p in LDS, a quarter of the dimensions.
+constexpr int kShareWaves = 4, kShareThreads = 64 * kShareWaves;
+
+// LDS of the statistics: each wave's two half-blocks of keys, the block sums.
+template <int D>
+constexpr size_t share_stats_lds(int tiles) {
+    return (size_t)kShareWaves * 2 * 32 * D * 2 + (size_t)tiles * 16 * 4;
+}
+
+template <int D, bool LONG>
+__global__ __launch_bounds__(kShareThreads, 2) void share_stats_kernel(const FlashArgs f, float2* stats) {
+    extern __shared__ __align__(16) uint16_t sm[];
+    __shared__ float mx[kShareWaves][16];
+    constexpr int U = D / 8, LPH = 32 * U / 64;  // wave loads of a half-block
+    const int lane = threadIdx.x & 63, j = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = blockIdx.x, g = h / (f.heads / f.kv_heads), q0 = (gridDim.y - 1 - blockIdx.y) * 16;
+    const int qrow = q0 + (lane & 15), qpos = f.p0 + qrow, first = f.p0 + q0, last = f.p0 + f.rows - 1;
+    const bool in = qrow < f.rows;
+    const int tiles = (min(first + 16, f.p0 + f.rows) + kBlockKeys - 1) / kBlockKeys;
+    const uint16_t* K = f.kv_base + (((size_t)f.layer * 2) * f.kv_heads + g) * (size_t)f.cap * D;
+    uint16_t* ks = sm + wave * 2 * 32 * D;
+    float* us = reinterpret_cast<float*>(sm + kShareWaves * 2 * 32 * D);  // [tile][query]
+    float qf[D / 8][2];
+    load_query<D>(f.q + ((size_t)min(qrow, f.rows - 1) * f.heads + h) * D, in, qf);
+    auto stage = [&](int t, int half) {
+#pragma unroll
+        for (int i = 0; i < LPH; ++i) {
+            const int u = i * 64 + lane, key = u / U, c = (u % U) ^ key_swz<D>(key);
+            __builtin_amdgcn_global_load_lds(
+                (Y2_GLOBAL void*)(K + (size_t)min(t * kBlockKeys + half * 32 + key, last) * D + 8 * c),
+                (lds_void*)(ks + half * 32 * D + i * 512), 16, 0, 0);
+        }
     };
-    if (head_dim == 128 && !lng) run(rows_stats_kernel<128, false>, rows_pv_kernel<128, false>);
-    else if (head_dim == 128) run(rows_stats_kernel<128, true>, rows_pv_kernel<128, true>);
-    else if (head_dim == 64 && !lng) run(rows_stats_kernel<64, false>, rows_pv_kernel<64, false>);
-    else if (head_dim == 64) run(rows_stats_kernel<64, true>, rows_pv_kernel<64, true>);
+    const int mine = tiles > wave ? (tiles - wave + kShareWaves - 1) / kShareWaves : 0;  // tiles wave, wave + 4, ..
+    float m = -__builtin_huge_valf();
+    for (int pass = 0; pass < 2; ++pass) {
+        if (mine > 0) stage(wave, 0);
+        for (int i = 0; i < mine; ++i) {
+            const int t = wave + kShareWaves * i, kb = t * kBlockKeys;
+            const bool masked = kb + kBlockKeys - 1 > first;
+            f32x4 s[4];
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                // this half has landed, the other one's reads are done
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                if (half == 0) stage(t, 1);
+                else if (i + 1 < mine) stage(t + kShareWaves, 0);
+                f32x4 v[2];
+                half_scores<D>(ks + half * 32 * D, qf, v);
+                s[2 * half] = v[0];
+                s[2 * half + 1] = v[1];
+            }
+            if (pass == 0) {
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (!masked || kb + kt * 16 + 4 * j + e <= qpos) m = fmaxf(m, s[kt][e]);
+                continue;
+            }
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float x = exp_nonpos(s[kt][e] * f.scale - m);
+                    s[kt][e] = !masked || kb + kt * 16 + 4 * j + e <= qpos ? x : 0.0f;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = xor_sum<32, 16>((s[0][e] + s[2][e]) + (s[1][e] + s[3][e]));
+            if (j == 0) us[t * 16 + (lane & 15)] = (v[0] + v[2]) + (v[1] + v[3]);
+        }
+        if (pass == 0) {
+            m = xor_max<32, 16>(m);
+            if (j == 0) mx[wave][lane & 15] = m;
+            __syncthreads();
+            m = mx[0][lane & 15];
+#pragma unroll
+            for (int w = 1; w < kShareWaves; ++w) m = fmaxf(m, mx[w][lane & 15]);
+            m = m * f.scale;  // the scaled maximum (rounding is monotonic)
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 16 && in) {
+        const int nb = (qpos + kBlockKeys) / kBlockKeys;
+        const bool two = LONG && nb >= 256;
+        float total = us[lane];
+        if (two) {
+            total = us[lane] + us[16 + lane];
+            for (int t = 2; t < nb; t += 2) total = total + (t + 1 < nb ? us[t * 16 + lane] + us[t * 16 + 16 + lane] : us[t * 16 + lane]);
+        } else {
+            for (int t = 1; t < nb; ++t) total = total + us[t * 16 + lane];
+        }
+        stats[(size_t)qrow * f.heads + h] = make_float2(m, total);
+    }
+}
+
+template <int D, bool LONG>
+__global__ __launch_bounds__(kShareThreads, 2) void share_pv_kernel(const FlashArgs f, const float2* stats) {
+    constexpr int VU = kBlockKeys / 2 * (D / 8), VS = VU / kShareThreads > 0 ? VU / kShareThreads : 1;
+    constexpr int DW = D / 16 / kShareWaves;  // 16-dim tiles per wave
+    static_assert(VU % kShareThreads == 0 && DW >= 1, "whole units and tiles");
+    __shared__ __align__(16) uint16_t ks[2][kBlockKeys * D];
+    __shared__ __align__(16) uint16_t vt[2][D * kBlockKeys];  // as in rows_pv_kernel
+    __shared__ __align__(16) f32x4 ps[2][kShareWaves][64];    // p of keys 16 kt + 4 j .. + 3, wave kt's lane
+    const int tid = threadIdx.x, lane = tid & 63, j = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = blockIdx.x, g = h / (f.heads / f.kv_heads), q0 = (gridDim.y - 1 - blockIdx.y) * 16;
+    const int qrow = q0 + (lane & 15), qpos = f.p0 + qrow, last = f.p0 + f.rows - 1;
+    const bool in = qrow < f.rows;
+    const int nt = (min(f.p0 + q0 + 16, f.p0 + f.rows) + kBlockKeys - 1) / kBlockKeys, tiles = LONG ? (nt + 1) & ~1 : nt;
+    const bool two = LONG && (qpos + kBlockKeys) / kBlockKeys >= 256;
+    const uint16_t* K = f.kv_base + (((size_t)f.layer * 2) * f.kv_heads + g) * (size_t)f.cap * D;
+    const uint16_t* V = f.kv_base + (((size_t)f.layer * 2 + 1) * f.kv_heads + g) * (size_t)f.cap * D;
+    float qf[D / 8][2];
+    load_query<D>(f.q + ((size_t)min(qrow, f.rows - 1) * f.heads + h) * D, in, qf);
+    const float2 mt = in ? stats[(size_t)qrow * f.heads + h] : make_float2(0.0f, 1.0f);
+    f32x4 o[DW], pend[DW];
+#pragma unroll
+    for (int d = 0; d < DW; ++d) o[d] = pend[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    uint4 va[VS], vb[VS];
+    auto load_values = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < VS; ++i) {
+            const int u = tid + kShareThreads * i, k = t * kBlockKeys + 2 * (u % (kBlockKeys / 2));
+            const int vd = u / (kBlockKeys / 2) * 8;
+            va[i] = ldg4(V + (size_t)min(k, last) * D + vd);
+            vb[i] = ldg4(V + (size_t)min(k + 1, last) * D + vd);
+        }
+    };
+    stage_keys<D, kShareWaves>(K, 0, last, ks[0]);
+    load_values(0);
+    for (int t = 0; t < tiles; ++t) {
+        const int kb = t * kBlockKeys, buf = t & 1;
+#pragma unroll
+        for (int i = 0; i < VS; ++i) {
+            const int u = tid + kShareThreads * i, vd = u / (kBlockKeys / 2) * 8;
+            const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), at = ((k >> 4) & 1) * 4 + (k & 3);
+            const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, b[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int d = vd + e;
+                const uint32_t w = e & 1 ? (a[e >> 1] >> 16) | (b[e >> 1] & 0xffff0000u)
+                                         : (a[e >> 1] & 0xffffu) | (b[e >> 1] << 16);
+                *reinterpret_cast<uint32_t*>(&vt[buf][d * kBlockKeys + ((unit ^ ((d >> 1) & 7)) << 3) + at]) = w;
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        asm volatile("s_barrier" ::: "memory");  // block t is staged; block t - 1's scores and p are read
+        if (t + 1 < tiles) {
+            stage_keys<D, kShareWaves>(K, t + 1, last, ks[buf ^ 1]);
+            load_values(t + 1);
+        }
+        {
+            // the p of this wave's 16 keys (one tile of a half-block's two: the other is another wave's)
+            f32x4 s;
+            tile_scores<D>(ks[buf] + wave * 16 * D, qf, s);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x = exp_nonpos(s[e] * f.scale - mt.x) / mt.y;
+                s[e] = kb + wave * 16 + 4 * j + e <= qpos ? x : 0.0f;
+            }
+            ps[buf][wave][lane] = s;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        asm volatile("s_barrier" ::: "memory");  // every wave's p (the next block's loads stay in flight)
+        f32x4 p[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) p[kt] = ps[buf][kt][lane];
+#pragma unroll
+        for (int d = 0; d < DW; ++d) {
+            const f32x4 v = pv_tile<D>(&vt[buf][((wave * DW + d) * 16 + (lane & 15)) * kBlockKeys], p);
+            if constexpr (!LONG) {
+                o[d] = t == 0 ? v : o[d] + v;
+            } else if (t & 1) {
+                const f32x4 pair = pend[d] + v, a = o[d] + pair, b = (o[d] + pend[d]) + v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[d][e] = t == 1 ? pair[e] : two ? a[e] : b[e];
+            } else {
+                pend[d] = v;
+            }
+        }
+    }
+    if (in) {
+        uint16_t* orow = f.out + ((size_t)qrow * f.heads + h) * D + 4 * j;
+#pragma unroll
+        for (int d = 0; d < DW; ++d) {
+            const uint32_t w0 = (uint32_t)bf16_bits(rb(o[d][0])) | ((uint32_t)bf16_bits(rb(o[d][1])) << 16);
+            const uint32_t w1 = (uint32_t)bf16_bits(rb(o[d][2])) | ((uint32_t)bf16_bits(rb(o[d][3])) << 16);
+            *reinterpret_cast<uint2*>(orow + (wave * DW + d) * 16) = make_uint2(w0, w1);
+        }
+    }
+}
+
+template <int D, bool LONG>
+static void rows_attention_t(hipStream_t s, const FlashArgs& f, float2* stats) {
+    if (LONG && (long)f.heads * ((f.rows + kRowsQ - 1) / kRowsQ) >= 256) {
+        const dim3 grid(f.heads, (f.rows + kRowsQ - 1) / kRowsQ);
+        rows_stats_kernel<D><<<grid, kRowsThreads, 0, s>>>(f, stats);
+        rows_pv_kernel<D><<<grid, kRowsThreads, 0, s>>>(f, stats);
+        return;
+    }
+    const dim3 grid(f.heads, (f.rows + 15) / 16);
+    const size_t lds = share_stats_lds<D>((f.p0 + f.rows + kBlockKeys - 1) / kBlockKeys);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&share_stats_kernel<D, LONG>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+    (void)attr;  // (a refusal shows at the launch)
+    share_stats_kernel<D, LONG><<<grid, kShareThreads, lds, s>>>(f, stats);
+    share_pv_kernel<D, LONG><<<grid, kShareThreads, 0, s>>>(f, stats);
+}
+
+hipError_t launch_rows_attention(hipStream_t s, const FlashArgs& f, float2* stats, int head_dim) {
+    const bool lng = f.p0 + f.rows > kLongKeys;
+    if (head_dim == 128) lng ? rows_attention_t<128, true>(s, f, stats) : rows_attention_t<128, false>(s, f, stats);
+    else if (head_dim == 64) lng ? rows_attention_t<64, true>(s, f, stats) : rows_attention_t<64, false>(s, f, stats);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -643,15 +896,15 @@ bool rows_supported(const Yue2Model* m, int context, int n) {
     if (n < 2 || (c.head_dim != 64 && c.head_dim != 128)) return false;
     if (c.hidden_size % kGemmTK || c.intermediate_size % kGemmTK || (c.num_attention_heads * c.head_dim) % kGemmTK)
         return false;
-    // A token step costs about the same whatever n is, and spreads a long
-    // context's keys over the chip; here each wave walks all of them.
-    // Measured, four 3B-class layers and the head (us): 950 + 1.27 per cached
+    // A token step costs about the same whatever n is; here few rows cost as
+    // much as 32, and their attention walks the context with few workgroups.
+    // Measured, four 3B-class layers and the head (us): 880 + 0.38 per cached
     // key against 200 + 230 n (265 n at 8000 keys); two layers of the reduced
-    // shape: 230 + 0.41 against 65 + 75 n; four of the YuE2 shape: 820 + 1.27
-    // against 240 + 175 n (195 n); four of a 1B class: 770 + 0.85 against
-    // 160 + 215 n.  The lines cross at n = 3-4 without a context, 10-18 at
-    // 2048 keys, 34-55 at 8000.
-    return n >= 4 + context / 150;
+    // shape: 200 + 0.11 against 65 + 73 n; four of the YuE2 shape: 770 + 0.36
+    // against 240 + 175 n (195 n); four of a 1B class: 720 + 0.24 against
+    // 160 + 215 n.  The lines cross at n = 3-4 without a context, 5-7 at 2048
+    // keys, 12-17 at 8000.
+    return n >= 4 + (context + 299) / 600;
 }
 
 int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, bool head) {
