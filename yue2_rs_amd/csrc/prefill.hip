@@ -80,6 +80,9 @@ struct GemmTile {
 // 128 x 64 and 64 x 64 wave blocks, four-wave tiles and 32-wide K steps.)
 using GemmBig = GemmTile<256, 256, 4, 2, 2>;
 using GemmNarrow = GemmTile<128, 256, 2, 4, 3>;
+// 192 x 256, 8 waves of 96 x 64: between the two, for grids whose last round
+// of the larger tile would be nearly empty.
+using GemmMid = GemmTile<192, 256, 2, 4, 2>;
 
 __device__ __forceinline__ int gemm_swz(int row) { return (row >> 1) & 7; }
 __device__ __forceinline__ int gemm_unit(int row, int c) { return row * 8 + (c ^ gemm_swz(row)); }
@@ -256,6 +259,11 @@ __global__ __launch_bounds__(T::THREADS, 1) void gemm_kernel(const GemmArgs g) {
     }
 }
 
+// What a row of a tile's round costs against the 256-row tile's, in percent
+// (from 24000 x 3072 x 3072 and x 8192, where every CU is busy for rounds: 442
+// and 1077 us, 447 and 1107 with the 192-row tile, 502 and 1246 with the 128).
+constexpr int kGemmMidWeight = 112, kGemmNarrowWeight = 126;
+
 template <int EPI, class T>
 static hipError_t launch_gemm_t(hipStream_t s, const GemmArgs& g) {
     // more than the default 64 KiB of dynamic LDS: allowed once per kernel
@@ -270,7 +278,6 @@ static hipError_t launch_gemm_t(hipStream_t s, const GemmArgs& g) {
 
 template <int EPI>
 static hipError_t launch_gemm_e(hipStream_t s, const GemmArgs& g) {
-    // the 256 x 256 tile unless its grid would fill fewer than half the CUs
     static const int cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -278,9 +285,21 @@ static hipError_t launch_gemm_e(hipStream_t s, const GemmArgs& g) {
             n = 256;
         return n;
     }();
-    const int tn = EPI == GEPI_SWIGLU_BF16 ? GemmBig::TW / 2 : GemmBig::TW;
-    const long tiles = (long)((g.N + tn - 1) / tn) * ((g.M + GemmBig::TM - 1) / GemmBig::TM);
-    return 2 * tiles >= cus ? launch_gemm_t<EPI, GemmBig>(s, g) : launch_gemm_t<EPI, GemmNarrow>(s, g);
+    // One workgroup runs per CU, so a grid takes whole rounds of a tile's
+    // time: the tile with the least rounds x rows, the smaller ones' rows
+    // counted dearer for their extra operand reads per MFMA.  Against the
+    // 256-row tile wherever it fills half the CUs and else the 128-row one,
+    // us: 2048 x 5120 x 3072 77 -> 69, 4096 156 -> 137; 3003 x 3072 x 3072 78
+    // -> 66, x 8192 189 -> 166, 6000 156 -> 132 and 371 -> 315; the pair at
+    // 517 x 8192 x 3072 95 -> 76.
+    const int tn = EPI == GEPI_SWIGLU_BF16 ? 128 : 256;
+    auto cost = [&](int tm, int weight) {
+        const long tiles = (long)((g.N + tn - 1) / tn) * ((g.M + tm - 1) / tm);
+        return (tiles + cus - 1) / cus * tm * weight;
+    };
+    const long big = cost(256, 100), mid = cost(192, kGemmMidWeight), narrow = cost(128, kGemmNarrowWeight);
+    if (big <= mid && big <= narrow) return launch_gemm_t<EPI, GemmBig>(s, g);
+    return mid <= narrow ? launch_gemm_t<EPI, GemmMid>(s, g) : launch_gemm_t<EPI, GemmNarrow>(s, g);
 }
 
 hipError_t launch_gemm(hipStream_t s, int epi, const GemmArgs& g) {
