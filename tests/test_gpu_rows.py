@@ -97,6 +97,45 @@ def test_many_rows_equal_token_steps(shape, context, n):
         _check(gm, context, rows - 128 + n, seed=n)
 
 
+# (head_dim, context, rows, position of the id whose value overflows): in the
+# middle of a wave's queries and of a block; in the last row of a block; in
+# the kernels of long contexts, with rows on both sides of the 256th block
+@pytest.mark.parametrize("head_dim,context,n,at", [(64, 0, 83, 70), (128, 0, 83, 70), (64, 5, 200, 122), (128, 5, 40, 30),
+                                                   (64, 15000, 2048, 1400), (128, 15000, 2048, 1400)])
+def test_rows_before_an_infinite_value(gpu, head_dim, context, n, at):
+    """A row attends the keys up to its own: what is computed for it does not
+    depend on the ids after it, also where a later id's value row overflows
+    to infinity (0 * inf would be NaN)."""
+    cfg = _config(1024, 16, 4, head_dim, 512, vocab=64)
+    ck = synthetic.checkpoint(cfg, seed=3)
+    # component 0 of the embedding: only id 63 has one, its only one, and it
+    # overflows dimension 0 of its value in the first layer
+    embed = ck.embed_tokens.reshape(cfg.vocab_size, -1)
+    embed[:, 0] = 0
+    embed[63] = 0
+    embed[63, 0] = 0x3f80
+    v = ck.layers[0].v_proj.reshape(-1, cfg.hidden_size)
+    v[:] = 0
+    v[0, 0] = 0x7f00  # 1.7e38; the norm makes the component 32
+    rng = np.random.default_rng(n)
+    v[1:, 1:] = (rb(0.02 * rng.standard_normal(v[1:, 1:].shape)).view(np.uint32) >> 16).astype(np.uint16)
+    gm = y2.Model.open(ck)
+    ids = np.asarray(synthetic.prompt(n, 63, 4), np.int32)
+    print(f"head_dim {head_dim}, context {context}, {n} ids", flush=True)
+    rows = []
+    for special in (63, 7):
+        ids[at] = special
+        c = _filled(gm, context, context + n, 2)
+        gm.forward_phase(ids, c, 0)
+        rows.append([a[:, context:] for a in c.export(context, n)])
+        c.close()
+    gm.close()
+    assert np.isinf(rows[0][1][0, at, 0]) and not np.isfinite(rows[0][0][1, at]).any(), "the id does not overflow"
+    for x, y in zip(*rows):
+        assert np.isfinite(y[:, :at]).all()
+        assert np.array_equal(bits(x[:, :at]), bits(y[:, :at])), "rows before the infinity differ"
+
+
 def test_prompt_equals_oracle(gpu, oracle_threads):
     ck = synthetic.checkpoint(SHAPES["d64"], seed=6)
     gm, om = y2.Model.open(ck), O.Model(ck)

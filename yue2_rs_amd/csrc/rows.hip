@@ -445,6 +445,77 @@ __device__ __forceinline__ f32x4 pv_tile(const uint16_t* vrow, const f32x4 (&p)[
     return (acc[0] + acc[2]) + (acc[1] + acc[3]);
 }
 
+// The same over the first `keys` keys of the block alone, on the vector ALU
+// (vt: the transposed V tile's first row of these 16 dims).  pv_tile
+// multiplies all of the block's keys, those past a query's last one with p =
+// 0 and (D = 64) each stream's with 0 in the other's pass, so an infinite or
+// NaN value makes NaN of sums that it does not belong to.  What it makes stays
+// in the output: the PV kernels walk the blocks a second time, this way, when
+// an output is not finite; ordinary values pay for a vote per workgroup and a
+// branch per block (2048 tokens, four 3B-class layers: 20.09 -> 20.18 ms).
+template <int D>
+__device__ __forceinline__ f32x4 pv_exact(const uint16_t* vt, const f32x4 (&p)[4], int keys) {
+    constexpr int SETS = D == 64 ? 2 : 1;  // streams e (and 4 + e): keys 16 kt + 4 j + e of every (second) j
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // (its addresses are not kept in registers from block to block)
+    const int d0 = (lane >> 4) * 4;
+    f32x4 part[2];
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int e2 = 0; e2 < 4; e2 += 2) {
+            const int e = e2 + half;
+            f32x4 sum;
+#pragma unroll
+            for (int set = 0; set < SETS; ++set) {
+                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) {
+                    const float mine = half ? p[kt][e2 + 1] : p[kt][e2];
+#pragma unroll
+                    for (int j = set; j < 4; j += SETS) {
+                        const float pk = __shfl(mine, (lane & 15) + 16 * j);
+                        const bool in = 16 * kt + 4 * j + e < keys;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int d = d0 + r, unit = (2 * j + (kt >> 1)) ^ ((d >> 1) & 7);
+                            const float v = bf16(vt[d * kBlockKeys + unit * 8 + (kt & 1) * 4 + e]);
+                            acc[r] = in ? __builtin_fmaf(v, pk, acc[r]) : acc[r];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                sum = set ? sum + acc : acc;
+            }
+            part[1] = e2 ? part[1] + sum : sum;
+        }
+        if (half == 0) part[0] = part[1];
+    }
+    return part[0] + part[1];
+}
+
+__device__ __forceinline__ bool finite(const f32x4& v) {
+    bool ok = true;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ok = ok && __builtin_fabsf(v[e]) <= 3.402823466e38f;
+    return ok;
+}
+
+// Whether v holds anywhere in a workgroup of NW waves; lds: NW words that no
+// wave uses between this call's barriers and the next one.
+template <int NW>
+__device__ __forceinline__ bool any_wave(bool v, uint16_t* lds) {
+    int* votes = reinterpret_cast<int*>(lds);
+    const bool mine = __builtin_amdgcn_ballot_w64(v) != 0;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) votes[threadIdx.x >> 6] = mine;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) any |= votes[w];
+    return any != 0;
+}
+
 // The DOTs of a block's 64 keys.
 template <int D>
 __device__ __forceinline__ void block_scores(const uint16_t* ks, const float (&qf)[D / 8][2], f32x4 (&s)[4]) {
@@ -597,58 +668,68 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_pv_kernel(const FlashArg
             }
         }
     };
-    stage_keys<D, kRowsWaves>(K, 0, last, ks[0]);
-    load_values(0);
-    for (int t = 0; t < tiles; ++t) {
-        const int kb = t * kBlockKeys, buf = t & 1;
+    for (bool exact = false;; exact = true) {
+        stage_keys<D, kRowsWaves>(K, 0, last, ks[0]);
+        load_values(0);
+        for (int t = 0; t < tiles; ++t) {
+            const int kb = t * kBlockKeys, buf = t & 1;
 #pragma unroll
-        for (int i = 0; i < VS; ++i) {
-            const int u = tid + kRowsThreads * i, vd = u / (kBlockKeys / 2) * 8;
-            if (u >= VU) continue;
-            const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), in = ((k >> 4) & 1) * 4 + (k & 3);
-            const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, b[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
+            for (int i = 0; i < VS; ++i) {
+                const int u = tid + kRowsThreads * i, vd = u / (kBlockKeys / 2) * 8;
+                if (u >= VU) continue;
+                const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), in = ((k >> 4) & 1) * 4 + (k & 3);
+                const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, b[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int d = vd + e;
-                const uint32_t w = e & 1 ? (a[e >> 1] >> 16) | (b[e >> 1] & 0xffff0000u)
-                                         : (a[e >> 1] & 0xffffu) | (b[e >> 1] << 16);
-                *reinterpret_cast<uint32_t*>(&vt[buf][d * kBlockKeys + ((unit ^ ((d >> 1) & 7)) << 3) + in]) = w;
+                for (int e = 0; e < 8; ++e) {
+                    const int d = vd + e;
+                    const uint32_t w = e & 1 ? (a[e >> 1] >> 16) | (b[e >> 1] & 0xffff0000u)
+                                             : (a[e >> 1] & 0xffffu) | (b[e >> 1] << 16);
+                    *reinterpret_cast<uint32_t*>(&vt[buf][d * kBlockKeys + ((unit ^ ((d >> 1) & 7)) << 3) + in]) = w;
+                }
             }
-        }
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        asm volatile("s_barrier" ::: "memory");  // block t is staged, block t - 1 read by every wave
-        if (t + 1 < tiles) {
-            stage_keys<D, kRowsWaves>(K, t + 1, last, ks[buf ^ 1]);
-            load_values(t + 1);
-        }
-        const bool live = kb <= r.wave_last;
-        f32x4 p[4];
-        if (live) {
-            block_scores<D>(ks[buf], qf, p);
-            const bool masked = kb + kBlockKeys - 1 > r.wave_first;
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            asm volatile("s_barrier" ::: "memory");  // block t is staged, block t - 1 read by every wave
+            if (t + 1 < tiles) {
+                stage_keys<D, kRowsWaves>(K, t + 1, last, ks[buf ^ 1]);
+                load_values(t + 1);
+            }
+            const bool live = kb <= r.wave_last;
+            f32x4 p[4];
+            if (live) {
+                block_scores<D>(ks[buf], qf, p);
+                const bool masked = kb + kBlockKeys - 1 > r.wave_first;
 #pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
+                for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float x = exp_nonpos(p[kt][e] * f.scale - mt.x) / mt.y;
-                    p[kt][e] = !masked || kb + kt * 16 + 4 * j + e <= r.qpos ? x : 0.0f;
+                    for (int e = 0; e < 4; ++e) {
+                        const float x = exp_nonpos(p[kt][e] * f.scale - mt.x) / mt.y;
+                        p[kt][e] = !masked || kb + kt * 16 + 4 * j + e <= r.qpos ? x : 0.0f;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) {
+                f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (__builtin_expect(exact, false)) {
+                    if (live) v = pv_exact<D>(&vt[buf][dt * 16 * kBlockKeys], p, r.qpos + 1 - kb);
+                } else {
+                    if (live) v = pv_tile<D>(&vt[buf][(dt * 16 + (lane & 15)) * kBlockKeys], p);
                 }
                 __builtin_amdgcn_sched_barrier(0);
+                if (t & 1) {
+                    const f32x4 pair = pend[dt] + v, a = o[dt] + pair, b = (o[dt] + pend[dt]) + v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[dt][e] = t == 1 ? pair[e] : two ? a[e] : b[e];
+                } else {
+                    pend[dt] = v;
+                }
             }
         }
+        bool ok = true;
 #pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) {
-            f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (live) v = pv_tile<D>(&vt[buf][(dt * 16 + (lane & 15)) * kBlockKeys], p);
-            __builtin_amdgcn_sched_barrier(0);
-            if (t & 1) {
-                const f32x4 pair = pend[dt] + v, a = o[dt] + pair, b = (o[dt] + pend[dt]) + v;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[dt][e] = t == 1 ? pair[e] : two ? a[e] : b[e];
-            } else {
-                pend[dt] = v;
-            }
-        }
+        for (int dt = 0; dt < D / 16; ++dt) ok = ok && finite(o[dt]);
+        if (exact || !any_wave<kRowsWaves>(r.in && !ok, vt[1])) break;
     }
     if (r.in) {
         uint16_t* orow = f.out + ((size_t)r.qrow * f.heads + r.h) * D + 4 * j;
@@ -765,7 +846,7 @@ __global__ __launch_bounds__(kShareThreads, 2) void share_stats_kernel(const Fla
 }
 
 template <int D, bool LONG>
-__global__ __launch_bounds__(kShareThreads, 2) void share_pv_kernel(const FlashArgs f, const float2* stats) {
+__global__ __launch_bounds__(kShareThreads, D == 64 && !LONG ? 4 : 2) void share_pv_kernel(const FlashArgs f, const float2* stats) {
     constexpr int VU = kBlockKeys / 2 * (D / 8), VS = VU / kShareThreads > 0 ? VU / kShareThreads : 1;
     constexpr int DW = D / 16 / kShareWaves;  // 16-dim tiles per wave
     static_assert(VU % kShareThreads == 0 && DW >= 1, "whole units and tiles");
@@ -796,58 +877,72 @@ __global__ __launch_bounds__(kShareThreads, 2) void share_pv_kernel(const FlashA
             vb[i] = ldg4(V + (size_t)min(k + 1, last) * D + vd);
         }
     };
-    stage_keys<D, kShareWaves>(K, 0, last, ks[0]);
-    load_values(0);
-    for (int t = 0; t < tiles; ++t) {
-        const int kb = t * kBlockKeys, buf = t & 1;
+    for (bool exact = false;; exact = true) {
+        stage_keys<D, kShareWaves>(K, 0, last, ks[0]);
+        load_values(0);
+        for (int t = 0; t < tiles; ++t) {
+            const int kb = t * kBlockKeys, buf = t & 1;
 #pragma unroll
-        for (int i = 0; i < VS; ++i) {
-            const int u = tid + kShareThreads * i, vd = u / (kBlockKeys / 2) * 8;
-            const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), at = ((k >> 4) & 1) * 4 + (k & 3);
-            const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, b[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
+            for (int i = 0; i < VS; ++i) {
+                const int u = tid + kShareThreads * i, vd = u / (kBlockKeys / 2) * 8;
+                const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), at = ((k >> 4) & 1) * 4 + (k & 3);
+                const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, b[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int d = vd + e;
-                const uint32_t w = e & 1 ? (a[e >> 1] >> 16) | (b[e >> 1] & 0xffff0000u)
-                                         : (a[e >> 1] & 0xffffu) | (b[e >> 1] << 16);
-                *reinterpret_cast<uint32_t*>(&vt[buf][d * kBlockKeys + ((unit ^ ((d >> 1) & 7)) << 3) + at]) = w;
+                for (int e = 0; e < 8; ++e) {
+                    const int d = vd + e;
+                    const uint32_t w = e & 1 ? (a[e >> 1] >> 16) | (b[e >> 1] & 0xffff0000u)
+                                             : (a[e >> 1] & 0xffffu) | (b[e >> 1] << 16);
+                    *reinterpret_cast<uint32_t*>(&vt[buf][d * kBlockKeys + ((unit ^ ((d >> 1) & 7)) << 3) + at]) = w;
+                }
             }
-        }
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        asm volatile("s_barrier" ::: "memory");  // block t is staged; block t - 1's scores and p are read
-        if (t + 1 < tiles) {
-            stage_keys<D, kShareWaves>(K, t + 1, last, ks[buf ^ 1]);
-            load_values(t + 1);
-        }
-        {
-            // the p of this wave's 16 keys (one tile of a half-block's two: the other is another wave's)
-            f32x4 s;
-            tile_scores<D>(ks[buf] + wave * 16 * D, qf, s);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float x = exp_nonpos(s[e] * f.scale - mt.x) / mt.y;
-                s[e] = kb + wave * 16 + 4 * j + e <= qpos ? x : 0.0f;
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            asm volatile("s_barrier" ::: "memory");  // block t is staged; block t - 1's scores and p are read
+            if (t + 1 < tiles) {
+                stage_keys<D, kShareWaves>(K, t + 1, last, ks[buf ^ 1]);
+                load_values(t + 1);
             }
-            ps[buf][wave][lane] = s;
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        asm volatile("s_barrier" ::: "memory");  // every wave's p (the next block's loads stay in flight)
-        f32x4 p[4];
+            {
+                // the p of this wave's 16 keys (one tile of a half-block's two: the other is another wave's)
+                f32x4 s;
+                tile_scores<D>(ks[buf] + wave * 16 * D, qf, s);
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) p[kt] = ps[buf][kt][lane];
+                for (int e = 0; e < 4; ++e) {
+                    const float x = exp_nonpos(s[e] * f.scale - mt.x) / mt.y;
+                    s[e] = kb + wave * 16 + 4 * j + e <= qpos ? x : 0.0f;
+                }
+                ps[buf][wave][lane] = s;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            asm volatile("s_barrier" ::: "memory");  // every wave's p (the next block's loads stay in flight)
+            f32x4 p[4];
 #pragma unroll
-        for (int d = 0; d < DW; ++d) {
-            const f32x4 v = pv_tile<D>(&vt[buf][((wave * DW + d) * 16 + (lane & 15)) * kBlockKeys], p);
-            if constexpr (!LONG) {
-                o[d] = t == 0 ? v : o[d] + v;
-            } else if (t & 1) {
-                const f32x4 pair = pend[d] + v, a = o[d] + pair, b = (o[d] + pend[d]) + v;
+            for (int kt = 0; kt < 4; ++kt) p[kt] = ps[buf][kt][lane];
+            f32x4 vs[DW];
+            if (__builtin_expect(exact, false)) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[d][e] = t == 1 ? pair[e] : two ? a[e] : b[e];
+                for (int d = 0; d < DW; ++d) vs[d] = pv_exact<D>(&vt[buf][(wave * DW + d) * 16 * kBlockKeys], p, qpos + 1 - kb);
             } else {
-                pend[d] = v;
+#pragma unroll
+                for (int d = 0; d < DW; ++d) vs[d] = pv_tile<D>(&vt[buf][((wave * DW + d) * 16 + (lane & 15)) * kBlockKeys], p);
+            }
+#pragma unroll
+            for (int d = 0; d < DW; ++d) {
+                const f32x4 v = vs[d];
+                if constexpr (!LONG) {
+                    o[d] = t == 0 ? v : o[d] + v;
+                } else if (t & 1) {
+                    const f32x4 pair = pend[d] + v, a = o[d] + pair, b = (o[d] + pend[d]) + v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[d][e] = t == 1 ? pair[e] : two ? a[e] : b[e];
+                } else {
+                    pend[d] = v;
+                }
             }
         }
+        bool ok = true;
+#pragma unroll
+        for (int d = 0; d < DW; ++d) ok = ok && finite(o[d]);
+        if (exact || !any_wave<kShareWaves>(in && !ok, vt[1])) break;
     }
     if (in) {
         uint16_t* orow = f.out + ((size_t)qrow * f.heads + h) * D + 4 * j;
