@@ -457,8 +457,7 @@ int32_t yue2_hip_model_set_prefill(Yue2Model *m, int32_t mfma);
  * entry lets a test place launches at that point.  The model must have run a
  * step-kernel forward. */
 int32_t yue2_hip_model_advance_sequence(Yue2Model *m, int32_t add);
-/* Diagnostics: RMSNorm guard fallbacks of the token steps since the model was
- * opened (multi-row calls do not count theirs). */
+/* Diagnostics: RMSNorm guard fallbacks taken since the model was opened. */
 int32_t yue2_hip_norm_fallbacks(const Yue2Model *m);
 
 /* Diagnostics: time one of the decoder's own kernels with HIP events on the

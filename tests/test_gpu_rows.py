@@ -97,6 +97,27 @@ def test_many_rows_equal_token_steps(shape, context, n):
         _check(gm, context, rows - 128 + n, seed=n)
 
 
+@pytest.mark.parametrize("step_kernel", [True, False])
+def test_norm_fallbacks_counted(shape, step_kernel):
+    """yue2_hip_norm_fallbacks counts a prompt's rows as it counts token
+    steps."""
+    gm, n = shape[2], 301
+    ids = np.asarray(synthetic.prompt(n, gm.config.vocab_size, 9), np.int32)
+    logits = np.empty(gm.config.vocab_size, np.float32)
+    gm.set_step_kernel(step_kernel)
+    counts = []
+    for cuts in ([n], [1] * n):
+        c, before, at = y2.Cache(gm, n), gm.norm_fallbacks(), 0
+        for k in cuts:
+            last = logits.ctypes.data if at + k == n else None
+            assert y2.lib().yue2_hip_forward(gm._h, c._h, ids[at:].ctypes.data, k, 0, last) == 0
+            at += k
+        counts.append(gm.norm_fallbacks() - before)
+        c.close()
+    gm.set_step_kernel(True)
+    assert counts[0] == counts[1] > 0
+
+
 # (head_dim, context, rows, position of the id whose value overflows): in the
 # middle of a wave's queries and of a block; in the last row of a block; in
 # the kernels of long contexts, with rows on both sides of the 256th block

@@ -39,9 +39,10 @@ hipError_t launch_gemm(hipStream_t s, int epi, const GemmArgs& g);
 // x[r] = the embedding row of ids[r] as f32 for r < rows (ids in range).
 hipError_t launch_embed_rows(hipStream_t s, const uint16_t* embed, const int32_t* ids, float* x, int rows, int H);
 
-// out[r] = RMSNorm(x[r]) as BF16 for r < rows (x row stride H).
+// out[r] = RMSNorm(x[r]) as BF16 for r < rows (x row stride H); *fallbacks
+// (or null) grows by the rows that took the sequential chain.
 hipError_t launch_norm_rows(hipStream_t s, const float* x, const float* gamma, uint16_t* out, int rows, int H,
-                            float eps);
+                            float eps, int32_t* fallbacks = nullptr);
 
 // Per (row r, head): the per-head RMSNorm of q and k and rotate-half RoPE at
 // position p0 + r: q heads into q (BF16 [rows][heads][D]), k and v heads

@@ -338,7 +338,7 @@ __global__ __launch_bounds__(kRowThreads) void embed_rows_kernel(const uint16_t*
 // values per thread and access (H a multiple of 4; one each measured 200 us
 // at 24000 x 3072 against 104, 34 against 30 at 2048).
 __global__ __launch_bounds__(kRowThreads) void norm_rows_kernel(const float* x, const float* gamma, uint16_t* out,
-                                                                int H, float eps) {
+                                                                int H, float eps, int32_t* fallbacks) {
     extern __shared__ __align__(16) float xs[];
     const int r = blockIdx.x;
     const float* row = x + (size_t)r * H;
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kRowThreads) void norm_rows_kernel(const float* x, 
         for (int k = 0; k < 4; ++k) norm_partial_add(e[0], w[0], v[k], i + k, H);
     }
     float s[1];
-    norm_scales_from<kRowThreads, 1>(e, w, xs, H, eps, nullptr, s);
+    norm_scales_from<kRowThreads, 1>(e, w, xs, H, eps, fallbacks, s);
     for (int i = 4 * threadIdx.x; i < H; i += 4 * kRowThreads) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(xs + i), g = *reinterpret_cast<const f32x4*>(gamma + i);
         uint32_t o[4];
@@ -596,9 +596,9 @@ hipError_t launch_embed_rows(hipStream_t s, const uint16_t* embed, const int32_t
 }
 
 hipError_t launch_norm_rows(hipStream_t s, const float* x, const float* gamma, uint16_t* out, int rows, int H,
-                            float eps) {
+                            float eps, int32_t* fallbacks) {
     if (rows < 1) return hipSuccess;
-    norm_rows_kernel<<<rows, kRowThreads, sizeof(float) * H, s>>>(x, gamma, out, H, eps);
+    norm_rows_kernel<<<rows, kRowThreads, sizeof(float) * H, s>>>(x, gamma, out, H, eps, fallbacks);
     return hipGetLastError();
 }
 

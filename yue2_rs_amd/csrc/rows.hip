@@ -1028,6 +1028,10 @@ int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, b
     int32_t* dids = reinterpret_cast<int32_t*>(b.p + o_ids);
     hipStream_t s = m->stream;
     const float eps = cf.rms_norm_eps;
+    // the norms' fallbacks, counted as the token steps of this model count them
+    // (the step kernel leaves out the final norm's)
+    int32_t* fallbacks = &m->ws.st->norm_fallbacks;
+    launch_fill(s, reinterpret_cast<float*>(fallbacks), 1, 0.0f);
     hipError_t e = hipMemcpyAsync(dids, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, s);
     for (int p0 = 0; p0 < n && e == hipSuccess; p0 += (int)R) {
         const int rows = std::min((int)R, n - p0), pos = c->length + p0;
@@ -1037,21 +1041,21 @@ int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, b
             const RopeArgs ra{qkv, q, c->kv, c->capacity, l, Hq, Hkv, D, pos, L.q_norm, L.k_norm,
                               m->rope_cos, m->rope_sin, eps};
             const FlashArgs fa{q, c->kv, c->capacity, l, Hq, Hkv, pos, rows, 1.0f / std::sqrt((float)D), att};
-            e = launch_norm_rows(s, x, L.in_norm, h, rows, H, eps);
+            e = launch_norm_rows(s, x, L.in_norm, h, rows, H, eps, fallbacks);
             if (e == hipSuccess)
                 e = launch_dot_gemm(s, GEPI_ROUND, GemmArgs{h, H, L.wqkv, nullptr, H, qkv, nullptr, qkvw, rows, qkvw, H});
             if (e == hipSuccess) e = launch_rope_append(s, ra, rows);
             if (e == hipSuccess) e = launch_rows_attention(s, fa, stats, D);
             if (e == hipSuccess)
                 e = launch_dot_gemm(s, GEPI_RESID, GemmArgs{att, qw, L.wo, nullptr, qw, x, nullptr, H, rows, H, qw});
-            if (e == hipSuccess) e = launch_norm_rows(s, x, L.post_norm, h, rows, H, eps);
+            if (e == hipSuccess) e = launch_norm_rows(s, x, L.post_norm, h, rows, H, eps, fallbacks);
             if (e == hipSuccess)
                 e = launch_dot_gemm(s, GEPI_SWIGLU_BF16, GemmArgs{h, H, L.wg, L.wu, H, nullptr, act, I, rows, I, H});
             if (e == hipSuccess)
                 e = launch_dot_gemm(s, GEPI_RESID, GemmArgs{act, I, L.wd, nullptr, I, x, nullptr, H, rows, H, I});
         }
         if (e == hipSuccess && head && p0 + rows == n)
-            if (int rc = enqueue_head(m, m->ws, x + (size_t)(rows - 1) * H, phase, s)) {
+            if (int rc = enqueue_head(m, m->ws, x + (size_t)(rows - 1) * H, phase, s, 1, !m->step_kernel)) {
                 (void)hipStreamSynchronize(s);
                 return rc;
             }
@@ -1059,6 +1063,9 @@ int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, b
     const hipError_t done = hipStreamSynchronize(s);  // nothing runs over the scratch any more
     m->scratch.trim();
     if (e == hipSuccess) e = done;
+    int32_t taken = 0;
+    if (e == hipSuccess && hipMemcpy(&taken, fallbacks, sizeof(taken), hipMemcpyDeviceToHost) == hipSuccess)
+        m->norm_fallbacks += taken;
     return e == hipSuccess ? YUE2_OK : hip_fail(e, "multi-row forward");
 }
 

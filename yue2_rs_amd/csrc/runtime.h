@@ -163,8 +163,10 @@ bool device_ready();
 int enqueue_step(Yue2Model* m, Workspace& w, const KvView& kv, int rows, bool head, int phase,
                  hipStream_t s);
 // The final norm and the phase's LM head of `rows` rows x (stride hidden)
-// into w.logits (Model::forward_phase's projection, src/model.rs:469-507).
-int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStream_t s, int rows = 1);
+// into w.logits (Model::forward_phase's projection, src/model.rs:469-507);
+// count: the final norm's fallbacks are counted.
+int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStream_t s, int rows = 1,
+                 bool count = true);
 // The same step as one persistent kernel when the shape has one (full
 // vocabulary head only); returns 1 when it cannot be used.  sample: the
 // fused sampler's mode (StepCall::sample); the workspace must have been
