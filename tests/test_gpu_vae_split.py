@@ -54,3 +54,26 @@ def test_decode_with_both_tiles(gpu, tmp_path, frames):
     oracle = oracle_ops(cfg, t).run(z)
     assert np.abs(got - exact).max() <= 4 * np.abs(oracle - exact).max() + 1e-6
     vae.close()
+
+
+def _long_vae(seed, **kw):
+    cfg, t = synthetic_vae(seed=seed, channels=32, c_mults=(1, 2), strides=(4, 8), **kw)
+    return cfg, {n: a * np.float32(0.5) if n.endswith("weight_g") else a for n, a in t.items()}
+
+
+@pytest.mark.parametrize("arguments", ["ordinary", "large"])
+def test_tiles_equal_the_whole_decode(gpu, tmp_path, arguments):
+    """Tiles on the 64 x 64 kernel tile equal the whole decode, whose last
+    blocks take the 256 x 128 one, bit for bit; also where some of SnakeBeta's
+    arguments are past the range of its series (one channel, beside others in
+    the same wave)."""
+    cfg, t = _long_vae(12)
+    if arguments == "large":
+        for n in t:
+            if n.endswith(".alpha"):
+                t[n][3] = np.log(2e5)
+    vae = y2.Vae(write_vae_dir(tmp_path, cfg, t))
+    z = np.random.default_rng(8).standard_normal((1601, 16)).astype(np.float32)
+    full, tiled = vae.decode(z), vae.decode_tiled(z, 64, vae.required_halo(64))
+    vae.close()
+    assert np.array_equal(full.view(np.uint32), tiled.view(np.uint32))

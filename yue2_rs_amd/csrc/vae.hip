@@ -336,7 +336,8 @@ typedef __attribute__((address_space(3))) u32x2 lds_u32x2w;
 // sin(x)^2: x reduced by the nearest multiple of pi (two-part Cody-Waite; the
 // first difference is exact for |x| < 2^22), then the Taylor series of sin to
 // the 13th power on [-pi/2, pi/2] (remainder below 1e-9).  Past 1e5, and for
-// infinities, the library's sinf, decided by the wave.
+// infinities, the library's sinf (computed where a lane of the wave needs it
+// and taken by that lane alone: what shares a wave depends on the tiling).
 __device__ __forceinline__ float sin_squared(float x) {
     const float n = __builtin_rintf(x * 0.318309886f);
     float r = __builtin_fmaf(-n, 3.14159274101257324f, x);
@@ -349,7 +350,11 @@ __device__ __forceinline__ float sin_squared(float x) {
     q = __builtin_fmaf(q, z, 1.0f / 120.0f);
     q = __builtin_fmaf(q, z, -1.0f / 6.0f);
     float t = __builtin_fmaf(q * z, r, r);
-    if (__builtin_amdgcn_ballot_w64(!(__builtin_fabsf(x) <= 1e5f))) t = sinf(x);
+    const bool far = !(__builtin_fabsf(x) <= 1e5f);
+    if (__builtin_amdgcn_ballot_w64(far)) {
+        const float l = sinf(x);
+        t = far ? l : t;
+    }
     return t * t;
 }
 
