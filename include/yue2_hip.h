@@ -417,7 +417,8 @@ void yue2_hip_synthetic_bf16(uint16_t *out, size_t n, uint64_t seed, uint64_t te
  * 64-value vector, decided by one wave (stored on all 64 of its outputs);
  * 18 the RMSNorm scales of the two 128-value rows of each 256-value block,
  * decided together by a 256-thread block (each row's outputs hold its
- * scale).  Returns 0 or a negative Yue2Error. */
+ * scale); 19 sin(x)^2 as the VAE's SnakeBeta takes it, 20 the square of the
+ * device library's sinf.  Returns 0 or a negative Yue2Error. */
 int32_t yue2_hip_selftest_math(int32_t which, const void *in, void *out, size_t n);
 /* Diagnostics: out = x W^T (M x N f32, the raw FP32 accumulation) through
  * the prefill's BF16 MFMA GEMM; x [M, K] and w [N, K] BF16 host arrays, K a

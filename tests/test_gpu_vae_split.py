@@ -77,3 +77,38 @@ def test_tiles_equal_the_whole_decode(gpu, tmp_path, arguments):
     full, tiled = vae.decode(z), vae.decode_tiled(z, 64, vae.required_halo(64))
     vae.close()
     assert np.array_equal(full.view(np.uint32), tiled.view(np.uint32))
+
+
+def _sine_squared(which, x):
+    out = np.empty_like(x)
+    rc = y2.lib().yue2_hip_selftest_math(which, x.ctypes.data, out.ctypes.data, x.size)
+    assert rc == 0, y2.lib().yue2_hip_last_error().decode()
+    return out.astype(np.float64)
+
+
+@pytest.mark.parametrize("limit", [1.0, 10.0, 100.0, 1e4, 1e5])
+def test_sine_squared(gpu, limit):
+    """SnakeBeta's sin(x)^2 is no further from float64 than the square of the
+    library's sinf: in the largest and the root-mean-square difference, and in
+    the largest relative one, which multiples of pi and their neighbours
+    decide."""
+    rng = np.random.default_rng(int(limit))
+    n = 1 << 21
+    near = np.arange(1, int(limit / np.pi) + 1) * np.pi
+    near = np.resize(near, n // 2).astype(np.float32) if near.size else rng.uniform(0, limit, n // 2).astype(np.float32)
+    near = (near.view(np.int32) + rng.integers(-2, 3, near.size).astype(np.int32)).view(np.float32)
+    x = np.concatenate([rng.uniform(-limit, limit, n), limit * np.exp(rng.uniform(-20, 0, n // 2)), near])
+    x = x.astype(np.float32)
+    want = np.sin(x.astype(np.float64)) ** 2
+    measures = []
+    for which in (19, 20):
+        d = _sine_squared(which, x) - want
+        measures.append([np.abs(d).max(), np.sqrt(np.mean(d * d)), (np.abs(d) / np.maximum(want, 1e-300)).max()])
+    print(f"to {limit}: series {measures[0]}, sinf {measures[1]}", flush=True)
+    assert all(a <= b for a, b in zip(*measures))
+
+
+def test_sine_squared_of_what_is_not_finite(gpu):
+    x = np.resize(np.array([np.inf, -np.inf, np.nan, 0.0], np.float32), 256)
+    got = _sine_squared(19, x)
+    assert np.isnan(got[x != 0]).all() and (got[x == 0] == 0).all()

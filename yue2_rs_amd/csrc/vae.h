@@ -1,6 +1,7 @@
 // vae.h -- the VAE decoder (src/vae.rs) between its checkpoint reader
 // (checkpoint.hip) and its device executor (vae.hip).
 #pragma once
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <vector>
@@ -28,5 +29,9 @@ struct VaeHost {
 // safetensors file(s) of `dir`, checked as the reference checks them.
 // Returns 0 or a negative Yue2Error (message in yue2_hip_last_error).
 int vae_read(const char* dir, VaeHost* out);
+
+// out[i] = sin(in[i])^2 as SnakeBeta takes it (library: the square of sinf);
+// n a multiple of 4, 16-byte aligned.
+hipError_t launch_sine_selftest(hipStream_t s, const float* in, float* out, size_t n, bool library);
 
 }  // namespace y2

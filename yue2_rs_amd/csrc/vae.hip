@@ -333,29 +333,57 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) const y2_u32x4 lds_u32x4;
 typedef __attribute__((address_space(3))) u32x2 lds_u32x2w;
 
-// sin(x)^2: x reduced by the nearest multiple of pi (two-part Cody-Waite; the
-// first difference is exact for |x| < 2^22), then the Taylor series of sin to
-// the 13th power on [-pi/2, pi/2] (remainder below 1e-9).  Past 1e5, and for
-// infinities, the library's sinf (computed where a lane of the wave needs it
-// and taken by that lane alone: what shares a wave depends on the tiling).
-__device__ __forceinline__ float sin_squared(float x) {
-    const float n = __builtin_rintf(x * 0.318309886f);
-    float r = __builtin_fmaf(-n, 3.14159274101257324f, x);
-    r = __builtin_fmaf(-n, -8.74227766e-8f, r);
-    const float z = r * r;
-    float q = 1.0f / 6227020800.0f;
-    q = __builtin_fmaf(q, z, -1.0f / 39916800.0f);
-    q = __builtin_fmaf(q, z, 1.0f / 362880.0f);
-    q = __builtin_fmaf(q, z, -1.0f / 5040.0f);
-    q = __builtin_fmaf(q, z, 1.0f / 120.0f);
-    q = __builtin_fmaf(q, z, -1.0f / 6.0f);
-    float t = __builtin_fmaf(q * z, r, r);
-    const bool far = !(__builtin_fabsf(x) <= 1e5f);
-    if (__builtin_amdgcn_ballot_w64(far)) {
-        const float l = sinf(x);
-        t = far ? l : t;
+// sin(x)^2 of four values: x reduced by the nearest multiple n of pi/2
+// (three-part Cody-Waite, the first difference exact; n and its parity from
+// one addition to 1.5 * 2^23), sin(r)^2 = z + z^2 q(z) on [-pi/4, pi/4] with z
+// = r^2 and q a cubic fitted to the series (6.6e-9 of the result), one minus
+// it for odd n.  Past 1e5 the square of the library's sinf (computed where a
+// lane of the wave needs it and taken by that lane alone: what shares a wave
+// depends on the tiling; one branch for four values, so that their chains
+// interleave).  Against float64 up to 1e5: 1.02e-7 at most and 1.9e-8 rms,
+// within 2.6 ulp; the square of sinf 1.32e-7, 2.5e-8 and 3.1 ulp (the sine to
+// the 13th power on [-pi/2, pi/2], squared: 2.6e-7, 3.9e-8 and thousands of
+// ulp next to multiples of pi).
+__device__ __forceinline__ f32x4 sin_squared(const f32x4& x) {
+    f32x4 s;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float t = __builtin_fmaf(x[e], 0.636619772f, 12582912.0f), n = t - 12582912.0f;
+        float r = __builtin_fmaf(-n, 1.57079637050628662f, x[e]);
+        r = __builtin_fmaf(-n, -4.37113883e-8f, r);
+        r = __builtin_fmaf(-n, -1.71509942e-15f, r);
+        const float z = r * r;
+        float q = __builtin_fmaf(0x1.1ab602p-13f, z, -0x1.9fad96p-9f);
+        q = __builtin_fmaf(q, z, 0x1.6c1562p-5f);
+        q = __builtin_fmaf(q, z, -0x1.555552p-2f);
+        const float odd = u2f((uint32_t)((int32_t)(f2u(t) << 31) >> 31) & 0x3f800000u);
+        s[e] = __builtin_fabsf(odd - __builtin_fmaf(z * z, q, z));
     }
-    return t * t;
+    const float most = fmaxf(fmaxf(__builtin_fabsf(x[0]), __builtin_fabsf(x[1])),
+                             fmaxf(__builtin_fabsf(x[2]), __builtin_fabsf(x[3])));
+    if (__builtin_amdgcn_ballot_w64(most > 1e5f)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float l = sinf(x[e]);
+            s[e] = __builtin_fabsf(x[e]) > 1e5f ? l * l : s[e];
+        }
+    }
+    return s;
+}
+
+__global__ __launch_bounds__(256) void sine_selftest_kernel(const float* in, float* out, size_t n, int library) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (4 * i >= n) return;
+    const f32x4 x = *reinterpret_cast<const f32x4*>(in + 4 * i);
+    f32x4 s = sin_squared(x);
+    if (library) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float l = sinf(x[e]);
+            s[e] = l * l;
+        }
+    }
+    *reinterpret_cast<f32x4*>(out + 4 * i) = s;
 }
 
 // The three BF16 parts of two values, as pairs.
@@ -452,8 +480,9 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS == 512 ? 2 : 1) void conv_sp
         if (row >= span) return;
         f32x4 v = xr[s];
         if constexpr (ACT == ACT_SNAKE) {
+            const f32x4 t = sin_squared(v * ar);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = v[e] + br[e] * sin_squared(v[e] * ar[e]);
+            for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(br[e], t[e], v[e]);
         } else if constexpr (ACT == ACT_ELU) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = v[e] < 0.0f ? expf(v[e]) - 1.0f : v[e];
@@ -870,6 +899,12 @@ hipError_t run_conv(hipStream_t s, const VaeOpHost& op, const ConvShape& c, cons
 }
 
 }  // namespace
+
+hipError_t launch_sine_selftest(hipStream_t s, const float* in, float* out, size_t n, bool library) {
+    sine_selftest_kernel<<<(unsigned)((n + 1023) / 1024), 256, 0, s>>>(in, out, n, library);
+    return hipGetLastError();
+}
+
 }  // namespace y2
 
 struct Yue2Vae {
