@@ -15,7 +15,7 @@ from oracle import oracle as O
 import yue2_rs_amd as y2
 
 from test_gpu_vae import _selftest
-from vae_files import conv_case, decode_f64, oracle_ops, synthetic_vae, write_vae_dir
+from vae_files import conv_case, conv_f64, decode_f64, oracle_ops, synthetic_vae, write_vae_dir
 
 pytestmark = pytest.mark.gpu
 
@@ -112,3 +112,53 @@ def test_sine_squared_of_what_is_not_finite(gpu):
     x = np.resize(np.array([np.inf, -np.inf, np.nan, 0.0], np.float32), 256)
     got = _sine_squared(19, x)
     assert np.isnan(got[x != 0]).all() and (got[x == 0] == 0).all()
+
+
+HUGE = 3.4e38  # rounds to an infinite BF16 value
+# (place, value): the activation at (70, 5) or the weight of output 2, input 5, tap 1
+EXTREMES = [("x", np.inf), ("x", -np.inf), ("x", np.nan), ("x", HUGE), ("x", -HUGE), ("w", HUGE), ("w", -np.inf),
+            ("w", np.nan)]
+
+
+@pytest.mark.parametrize("place,value", EXTREMES)
+@pytest.mark.parametrize("shape", [(False, 32, 40, 7, 1, 3, 1, 200), (False, 32, 33, 1, 1, 0, 1, 100),
+                                   (True, 16, 64, 8, 4, 2, 1, 90), (False, 16, 32, 7, 1, 3, 1, 33000)])
+def test_extreme_operands(gpu, shape, place, value):
+    """Operands without finite BF16 parts give what FP32 arithmetic gives, and
+    the outputs that they do not enter stay as they are."""
+    transpose, cin, cout, kernel, stride, padding, dilation, frames = shape
+    x, w, b, plain = conv_case(*shape)
+    if place == "x":
+        x[70, 5] = value
+    else:
+        tap = min(1, kernel - 1)
+        w[(5, 2, tap) if transpose else (2, 5, tap)] = value
+    with np.errstate(all="ignore"):
+        want = conv_f64(transpose, x, w, b, kernel, stride, padding, dilation).astype(np.float32)
+    got = _selftest(transpose, cin, cout, kernel, stride, padding, dilation, x, w, b, want.shape[0])
+    same = np.abs(want - plain) < 1e30
+    assert not same.all() and np.abs(got - plain)[same].max() <= 1e-5
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~same & ~np.isnan(want)
+    assert np.array_equal(np.isinf(got[ok]), np.isinf(want[ok])) and np.array_equal(np.sign(got[ok]), np.sign(want[ok]))
+    ok &= np.isfinite(want)
+    # one product of full size: its rounding and those of the sum, which may
+    # round again after each of the few products that follow
+    assert (np.abs(got[ok] - want[ok]) <= 1e-6 * np.abs(want[ok])).all()
+
+
+def test_infinite_activations_through_the_last_tanh(gpu, tmp_path):
+    """An ELU decoder whose last unit overflows: its 1-tap convolution turns
+    one infinite input into infinities of both signs, ELU those into infinity
+    and -1, and the last convolution (weights of one sign) and tanh into
+    finite audio."""
+    cfg, t = _long_vae(13, snake=False)
+    last = max(int(n.split(".")[2]) for n in t if n.startswith("decoder.layers."))
+    t[f"decoder.layers.{last - 2}.layers.4.layers.1.bias"][0] = np.inf
+    name = f"decoder.layers.{last}.weight_v"
+    t[name] = np.abs(t[name])
+    vae = y2.Vae(write_vae_dir(tmp_path, cfg, t))
+    z = np.random.default_rng(8).standard_normal((40, 16)).astype(np.float32)
+    got = vae.decode(z)
+    vae.close()
+    assert (got == 1.0).all()

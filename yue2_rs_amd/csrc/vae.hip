@@ -53,6 +53,7 @@ constexpr int kMaxTaps = 8, kMaxPhases = 32;  // ConvPlan stays under the 4 KB k
 constexpr int kMmaTile = 128;
 constexpr int kChunk = 16, kNarrowRows = 256, kNarrowPad = 17;
 constexpr size_t kMaxLds = 160 * 1024;
+constexpr float kBf16Max = 0x1.fep+127f;
 enum { ACT_NONE = 0, ACT_SNAKE = 1, ACT_ELU = 2 };
 
 struct ConvPlan {
@@ -308,8 +309,12 @@ __global__ __launch_bounds__(256, 2) void conv_mfma_kernel(const ConvPlan p) {
 // of twice the length each.  Against float64 the six products are three times
 // closer than the FP32 chain (1024 x 1024 outputs: 0.35e-6 against 1.07e-6 at
 // 3584 terms, 0.17e-6 against 0.54e-6 at 896), since sixteen products enter
-// each rounding of the sum.  The parts cover the f32 range; an infinite value
-// gives NaN (SnakeBeta of an infinity already does).
+// each rounding of the sum.  The split is exact for 2^-100 <= |x| < 2^128 -
+// 2^119 (below, what denormal parts lose is under 2^-126; from there on the
+// first part would be infinite, where a weight's is the largest BF16 instead
+// and an activation's is).  Infinities, NaN and such activations leave the
+// accumulators they enter infinite or NaN, and an output that is not finite is
+// computed again as one FP32 chain (split_chain).
 //
 // Tile: TM = 32 MI WM output rows x TN = 32 NJ WN output channels, one tap of
 // 16 input channels per step.  The weights are split at load and laid out as
@@ -419,6 +424,50 @@ constexpr int split_slots(bool big, int nt) { return big ? (nt == 7 || nt == 2 ?
 template <class T>
 size_t split_lds(int nt, int span) {
     return (size_t)split_ring(nt) * T::STAGE * 2 + (size_t)2 * split_xc(nt) * 6 * span * 16;
+}
+
+// Output (m, o) of phase ph as one FP32 chain in conv_mfma_kernel's order (8
+// channels, tap, channel), over the source rows that there are; NaN ends it.
+template <int ACT>
+__device__ __forceinline__ float split_chain(const ConvPlan& p, int ph, int m, int o) {
+    const int c16s = p.cin / 16, nblk = p.cout_pad / 32, ntaps = p.ntaps[ph];
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int ch = 0; ch < p.cin && sum == sum; ch += 8) {
+#pragma unroll 1
+        for (int q = 0; q < ntaps; ++q) {
+            const int src = m + p.off[ph][q];
+            if (src < 0 || src >= p.rows_in) continue;
+            const uint16_t* w = reinterpret_cast<const uint16_t*>(p.w) +
+                                (((size_t)p.slab[ph][q] * c16s + ch / 16) * nblk + o / 32) * 3 * 512 +
+                                ((ch / 8 & 1) * 32 + o % 32) * 8;
+            const y2_u32x4 w0 = *reinterpret_cast<const y2_u32x4*>(w), w1 = *reinterpret_cast<const y2_u32x4*>(w + 512);
+            const y2_u32x4 w2 = *reinterpret_cast<const y2_u32x4*>(w + 1024);
+            f32x4 v[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                v[k] = *reinterpret_cast<const f32x4*>(p.x + (size_t)src * p.cin + ch + 4 * k);
+                if constexpr (ACT == ACT_SNAKE) {
+                    const f32x4 a = *reinterpret_cast<const f32x4*>(p.alpha + ch + 4 * k);
+                    const f32x4 b = *reinterpret_cast<const f32x4*>(p.inv_beta + ch + 4 * k), t = sin_squared(v[k] * a);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[k][e] = __builtin_fmaf(b[e], t[e], v[k][e]);
+                } else if constexpr (ACT == ACT_ELU) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[k][e] = v[k][e] < 0.0f ? expf(v[k][e]) - 1.0f : v[k][e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const int u = 2 * k + (e >> 1);
+                    const float a = e & 1 ? bf16_hi(w0[u]) : bf16_lo(w0[u]), b = e & 1 ? bf16_hi(w1[u]) : bf16_lo(w1[u]);
+                    sum = __builtin_fmaf(v[k][e], (a + b) + (e & 1 ? bf16_hi(w2[u]) : bf16_lo(w2[u])), sum);
+                }
+        }
+    }
+    return sum;
 }
 
 template <int ACT, int NT, class T>
@@ -578,6 +627,25 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS == 512 ? 2 : 1) void conv_sp
             asm volatile("s_barrier" ::: "memory");  // chunk ck + 1 is staged, chunk ck read by every wave
         }
     }
+    // the outputs to be computed again: 0 times a finite sum is 0
+    float zero = 0.0f;
+#pragma unroll
+    for (int i = 0; i < T::MI; ++i)
+#pragma unroll
+        for (int j = 0; j < T::NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) zero = __builtin_fmaf(acc[i][j][r], 0.0f, zero);
+    const bool again = __builtin_amdgcn_ballot_w64(!(zero == 0.0f)) != 0;
+    uint64_t which = 0;
+    if (__builtin_expect(again, false)) {
+#pragma unroll
+        for (int i = 0; i < T::MI; ++i)
+#pragma unroll
+            for (int j = 0; j < T::NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    which |= (uint64_t)!(__builtin_fabsf(acc[i][j][r]) <= 3.402823466e38f) << ((i * T::NJ + j) * 16 + r);
+    }
     const int ostride = p.ostride, o0 = p.o0[ph], cout = p.cout;
 #pragma unroll
     for (int i = 0; i < T::MI; ++i)
@@ -603,6 +671,20 @@ __global__ __launch_bounds__(T::THREADS, T::THREADS == 512 ? 2 : 1) void conv_sp
                 }
             }
         }
+    if (__builtin_expect(again, false)) {
+#pragma unroll 1
+        for (int k = 0; k < T::MI * T::NJ * 16; ++k) {
+            const int i = k / (T::NJ * 16), j = k / 16 % T::NJ, r = k % 16;
+            const int o = n0 + (wn * T::NJ + j) * 32 + l32;
+            const int m = m0 + (wm * T::MI + i) * 32 + 4 * h + 8 * (r >> 2) + (r & 3);
+            if (!(which >> k & 1) || m >= m_count || o >= cout) continue;
+            const size_t at = (size_t)(o0 + ostride * m) * cout + o;
+            float v = split_chain<ACT>(p, ph, m, o) + (p.b ? p.b[o] : 0.0f);
+            if (p.res) v = v + p.res[at];
+            if (p.tanh_out) v = tanhf(v);
+            p.y[at] = v;
+        }
+    }
 }
 
 // Weight slabs [k][cin_pad][CO]; one output row per thread.
@@ -736,9 +818,10 @@ std::vector<float> conv_slabs(const VaeOpHost& op, const ConvShape& c) {
                     const size_t frag = (((size_t)j * nchunks + i / 16) * (c.cout_pad / 32) + o / 32) * 3;
                     const size_t in = (size_t)((i % 16 / 8) * 32 + o % 32) * 8 + i % 8;
                     for (int part = 0; part < 3; ++part) {
-                        const float r = rb(v);
+                        float r = rb(v);
+                        if (std::isinf(r) && std::isfinite(v)) r = std::copysign(kBf16Max, v);
                         d[(frag + part) * 512 + in] = bf16_bits(r);
-                        v -= r;
+                        v = std::isfinite(r) ? v - r : 0.0f;
                     }
                 }
         return t;
