@@ -63,15 +63,18 @@ static std::vector<Yue2Model*> g_models;
 
 hipError_t device_malloc_bytes(void** p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipErrorOutOfMemory) return e;
-    bool freed = false;
-    for (Yue2Model* m : g_models) {
-        freed = freed || m->scratch.p;
-        m->scratch.release();
+    if (e == hipErrorOutOfMemory) {
+        bool freed = false;
+        for (Yue2Model* m : g_models) {
+            freed = freed || m->scratch.p;
+            m->scratch.release();
+        }
+        (void)hipGetLastError();
+        if (freed) e = hipMalloc(p, bytes);
     }
-    if (!freed) return e;
-    (void)hipGetLastError();
-    return hipMalloc(p, bytes);
+    // reported here: the next launch's check is not to find it
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 hipError_t Scratch::ensure(size_t want) {
