@@ -39,7 +39,12 @@ def _too_large_cache(gm):
         y2.Cache(gm, 2**31 - 1)
 
 
-@pytest.mark.parametrize("request_", [_too_large_cache], ids=["cache"])
+def _too_large_gemm(gm):
+    word = np.zeros(1, np.float32).ctypes.data
+    assert y2.lib().yue2_hip_selftest_gemm(word, word, word, 1 << 30, 1, 1 << 16) < 0
+
+
+@pytest.mark.parametrize("request_", [_too_large_cache, _too_large_gemm], ids=["cache", "selftest"])
 def test_scratch_given_back_to_a_failing_allocation(gpu, request_):
     gm = y2.Model.open(synthetic.checkpoint(synthetic.REDUCED, seed=0))
     ids = synthetic.prompt(16000, gm.config.vocab_size, 1)

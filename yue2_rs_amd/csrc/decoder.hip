@@ -480,7 +480,7 @@ extern "C" int32_t yue2_hip_decoder_time_kernel(Yue2Decoder* d, int32_t kernel, 
     const int rows = d->rows, L = c.num_hidden_layers;
     const size_t out_n = (size_t)rows * std::max(std::max(V, qkvw), std::max(I, H));
     float* tmp = nullptr;
-    hipError_t e = hipMalloc(&tmp, out_n * sizeof(float));
+    hipError_t e = device_malloc(&tmp, out_n * sizeof(float));
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(timing)");
     hipEvent_t b0, b1;
     (void)hipEventCreate(&b0);

@@ -40,7 +40,7 @@ struct DevBufs {
     std::vector<void*> p;
     void* alloc(size_t bytes) {
         void* q = nullptr;
-        if (hipMalloc(&q, bytes) != hipSuccess) return nullptr;
+        if (device_malloc(&q, bytes) != hipSuccess) return nullptr;
         p.push_back(q);
         return q;
     }

@@ -739,9 +739,9 @@ extern "C" int32_t yue2_hip_selftest_gemm(const uint16_t* x, const uint16_t* w, 
     if (!x || !w || !out || M < 1 || N < 1 || K < 1 || K % kGemmTK) return fail(YUE2_ERR_ARG, "bad gemm selftest");
     if (!device_ready()) return fail(YUE2_ERR_DEVICE, "no gfx950 device");
     void *dx = nullptr, *dw = nullptr, *dc = nullptr;
-    hipError_t e = hipMalloc(&dx, 2 * (size_t)M * K);
-    if (e == hipSuccess) e = hipMalloc(&dw, 2 * (size_t)N * K);
-    if (e == hipSuccess) e = hipMalloc(&dc, 4 * (size_t)M * N);
+    hipError_t e = device_malloc(&dx, 2 * (size_t)M * K);
+    if (e == hipSuccess) e = device_malloc(&dw, 2 * (size_t)N * K);
+    if (e == hipSuccess) e = device_malloc(&dc, 4 * (size_t)M * N);
     if (e == hipSuccess) e = hipMemcpy(dx, x, 2 * (size_t)M * K, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(dw, w, 2 * (size_t)N * K, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
@@ -778,9 +778,9 @@ extern "C" int32_t yue2_hip_bench_gemm(int32_t M, int32_t N, int32_t K, int32_t 
     if (!device_ready()) return fail(YUE2_ERR_DEVICE, "no usable gfx950 device");
     const int wrows = pair ? 2 * N : N;
     void *dx = nullptr, *dw = nullptr, *dc = nullptr;
-    hipError_t e = hipMalloc(&dx, 2 * (size_t)M * K);
-    if (e == hipSuccess) e = hipMalloc(&dw, 2 * (size_t)wrows * K);
-    if (e == hipSuccess) e = hipMalloc(&dc, 4 * (size_t)M * N);
+    hipError_t e = device_malloc(&dx, 2 * (size_t)M * K);
+    if (e == hipSuccess) e = device_malloc(&dw, 2 * (size_t)wrows * K);
+    if (e == hipSuccess) e = device_malloc(&dc, 4 * (size_t)M * N);
     if (e == hipSuccess) {
         bench_fill_kernel<<<1024, 256>>>(static_cast<uint16_t*>(dx), (size_t)M * K, 1);
         bench_fill_kernel<<<1024, 256>>>(static_cast<uint16_t*>(dw), (size_t)wrows * K, 2);

@@ -865,7 +865,7 @@ extern "C" int32_t yue2_hip_trace_step(Yue2Model* m, Yue2Cache* c, Yue2Cache* c2
     if (int rc = w.ensure(rows, blocks, m->c)) return rc;
     if (int rc = prepare_step(m, w)) return rc < 0 ? rc : fail(YUE2_ERR_ARG, "no step kernel for this shape");
     unsigned long long* dev = nullptr;
-    if (hipMalloc(&dev, n * sizeof(*dev)) != hipSuccess) return fail(YUE2_ERR_ALLOC, "trace buffer");
+    if (device_malloc(&dev, n * sizeof(*dev)) != hipSuccess) return fail(YUE2_ERR_ALLOC, "trace buffer");
     KvView kv{};
     for (int b = 0; b < rows; ++b) {
         kv.base[b] = cs[b]->kv;
@@ -910,8 +910,8 @@ extern "C" int32_t yue2_hip_selftest_math(int32_t which, const void* in, void* o
         return fail(YUE2_ERR_ARG, "bad selftest request");
     const size_t elem = which == 1 ? sizeof(double) : sizeof(float);
     void *din = nullptr, *dout = nullptr;
-    hipError_t e = hipMalloc(&din, n * elem);
-    if (e == hipSuccess) e = hipMalloc(&dout, n * elem);
+    hipError_t e = device_malloc(&din, n * elem);
+    if (e == hipSuccess) e = device_malloc(&dout, n * elem);
     if (e == hipSuccess) e = hipMemcpy(din, in, n * elem, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         if (which >= 19) {

@@ -1285,10 +1285,10 @@ extern "C" int32_t yue2_hip_selftest_conv(int32_t transpose, int32_t cin, int32_
     const ConvShape shape = conv_shape(op);
     const std::vector<float> slabs = conv_slabs(op, shape);
     float *dx = nullptr, *dw = nullptr, *db = nullptr, *dy = nullptr;
-    hipError_t e = hipMalloc(&dx, sizeof(float) * (size_t)frames * cin);
-    if (e == hipSuccess) e = hipMalloc(&dw, sizeof(float) * slabs.size());
-    if (e == hipSuccess) e = hipMalloc(&db, sizeof(float) * cout);
-    if (e == hipSuccess) e = hipMalloc(&dy, sizeof(float) * (size_t)len * cout);
+    hipError_t e = device_malloc(&dx, sizeof(float) * (size_t)frames * cin);
+    if (e == hipSuccess) e = device_malloc(&dw, sizeof(float) * slabs.size());
+    if (e == hipSuccess) e = device_malloc(&db, sizeof(float) * cout);
+    if (e == hipSuccess) e = device_malloc(&dy, sizeof(float) * (size_t)len * cout);
     if (e == hipSuccess) e = hipMemcpy(dx, x, sizeof(float) * (size_t)frames * cin, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(dw, slabs.data(), sizeof(float) * slabs.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess && bias) e = hipMemcpy(db, bias, sizeof(float) * cout, hipMemcpyHostToDevice);
