@@ -418,7 +418,12 @@ void yue2_hip_synthetic_bf16(uint16_t *out, size_t n, uint64_t seed, uint64_t te
  * 18 the RMSNorm scales of the two 128-value rows of each 256-value block,
  * decided together by a 256-thread block (each row's outputs hold its
  * scale); 19 sin(x)^2 as the VAE's SnakeBeta takes it, 20 the square of the
- * device library's sinf.  Returns 0 or a negative Yue2Error. */
+ * device library's sinf; 21 the exponential of the multi-row attention
+ * (arguments at most 0); 22, 23 eight-term dot products through FP32 MFMAs, the
+ * fma chain from +0 (a zero sum as +0), per group of inputs A [rows x 8] and B
+ * [columns x 8]: 22 16 x 16 outputs of 16x16x4 instructions, 23 the 16 rows of
+ * the group's parity of 32 x 32 outputs of 32x32x2 ones (n a multiple of 512).
+ * Returns 0 or a negative Yue2Error. */
 int32_t yue2_hip_selftest_math(int32_t which, const void *in, void *out, size_t n);
 /* Diagnostics: out = x W^T (M x N f32, the raw FP32 accumulation) through
  * the prefill's BF16 MFMA GEMM; x [M, K] and w [N, K] BF16 host arrays, K a

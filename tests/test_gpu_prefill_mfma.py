@@ -221,7 +221,8 @@ def test_full_depth_3b_against_decode_order_prefill(gpu):
 def test_full_depth_3b_24000_tokens_against_decode_order_prefill(gpu):
     """The long-context workload's prompt at full depth: 28 layers, 24000
     tokens, the MFMA prefill against the bit-exact decode-order GPU prefill
-    (24000 token steps), within the same full-depth bound; then the decode
+    (multi-row kernels, held to 24000 token steps on a smaller shape in
+    test_gpu_rows.py), within the same full-depth bound; then the decode
     step after it through each cache.  At this depth and length the two
     largest logits can sit closer than the bound (measured: a 0.17 std
     difference flipped the next step's argmax), so the argmax is reported,

@@ -7,7 +7,10 @@ oracle; the first case here is pinned to the oracle directly.  Sizes sit at
 the edges of the kernels: 16 queries per wave, 32-row tiles, 64-key blocks,
 128 rows per attention workgroup, contraction lengths of fewer than eight
 64-element lines and of a count that eight does not divide, the 256-block
-limit past which blocks are added in pairs."""
+limit past which blocks are added in pairs.  The instructions that this rests
+on are compared with the oracle's fma chains in themselves: the FP32 MFMAs over
+ordinary, wide-ranging and denormal operands, and the attention's own copy of
+the exponential."""
 import numpy as np
 import pytest
 
@@ -86,15 +89,34 @@ def test_long_append_equals_token_steps(shape, context, n):
         _check(shape[2], context, n, seed=context + n)
 
 
-# from 256 workgroups of 128 rows on, past 256 blocks: the attention kernels of
-# long contexts, their last workgroup with seven rows; and as many without a
-# context
-@pytest.mark.parametrize("context,n", [(0, 1), (13100, 7)])
+# from 256 workgroups of 128 rows on: as many as it takes, the last workgroup
+# with n rows.  Past 16320 keys they run the attention kernels of long
+# contexts: rows on both sides of the 256th block in one call (15000 cached
+# keys), or all of them past it, ending in an odd and in an even number of
+# blocks
+@pytest.mark.parametrize("context,n", [(0, 1), (15000, 7), (16300, 128), (16400, 60)])
 def test_many_rows_equal_token_steps(shape, context, n):
     name, _, gm = shape
     if name in ("d64", "d128"):
-        rows = 128 * (255 // gm.config.num_attention_heads + 1)
-        _check(gm, context, rows - 128 + n, seed=n)
+        heads = gm.config.num_attention_heads
+        rows = 128 * (255 // heads) + n
+        assert heads * -(-rows // 128) >= 256, "fewer workgroups than the long-context kernels are for"
+        assert context == 0 or context + rows > 255 * 64
+        _check(gm, context, rows, seed=n)
+
+
+def test_more_rows_than_a_pass_takes(shape):
+    """4096 rows go through the layers at a time: the second pass attends the
+    first one's rows."""
+    if shape[0] == "small":
+        _check(shape[2], 0, 4096 + 37, seed=3)
+
+
+def test_longest_prompt(shape):
+    """24000 ids in one call: six passes, the last of them in the kernels of
+    long contexts."""
+    if shape[0] == "d64":
+        _check(shape[2], 0, 24000, seed=6)
 
 
 @pytest.mark.parametrize("step_kernel", [True, False])
@@ -167,3 +189,44 @@ def test_prompt_equals_oracle(gpu, oracle_threads):
     for x, y in zip(cache.export(), oc.arrays()):
         assert np.array_equal(bits(x), bits(y[:, :83]))
     gm.close()
+
+
+def _selftest(which, x):
+    out = np.empty_like(x)
+    rc = y2.lib().yue2_hip_selftest_math(which, x.ctypes.data, out.ctypes.data, x.size)
+    assert rc == 0, y2.lib().yue2_hip_last_error().decode()
+    return out
+
+
+# operands: the exponents they are spread over
+@pytest.mark.parametrize("low,high", [(-1, 1), (-60, 60), (-80, -60), (-149, -120), (-149, 20)])
+@pytest.mark.parametrize("which,side,rows", [(22, 16, 16), (23, 32, 16)])
+def test_fp32_mfma_is_the_fma_chain(gpu, which, side, rows, low, high):
+    rng = np.random.default_rng(which + high + 200)
+    groups, n = 128, 2 * side * 8
+    x = (rng.uniform(1, 2, groups * n) * 2.0 ** rng.integers(low, high, groups * n)).astype(np.float32)
+    x *= rng.choice(np.array([-1, 1], np.float32), x.size)
+    x[rng.random(x.size) < 0.02] = 0.0
+    got = _selftest(which, x).reshape(groups, rows, side)
+    L = O.lib()
+    x = x.reshape(groups, 2, side, 8)
+    want = np.empty_like(got)
+    for g in range(groups):
+        for r in range(rows):
+            a = x[g, 0, r if side == rows else 2 * r + (g & 1)].ctypes.data
+            for c in range(side):
+                want[g, r, c] = L.y2o_dot_f32(a, x[g, 1, c].ctypes.data, 8)
+    assert np.array_equal(bits(got), bits(want))
+
+
+def test_attention_exponential(gpu):
+    """Every f32 from -2^-27 down to -128, and the ends, against the library's
+    other exponential, which test_gpu_math.py holds to the oracle's."""
+    lo, hi = (int(np.float32(-v).view(np.uint32)) for v in (2.0 ** -27, 128.0))
+    ends = np.array([0.0, -0.0, -1e-30, -1e-45, -150.0, -3e38, -np.inf, np.nan], np.float32)
+    for at in range(lo, hi, 1 << 26):
+        x = np.arange(at, at + (1 << 26), dtype=np.uint64).clip(lo, hi).astype(np.uint32).view(np.float32).copy()
+        x[:8] = ends
+        got, want = _selftest(21, x), _selftest(0, x)
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got), nan) and np.array_equal(bits(got)[~nan], bits(want)[~nan])

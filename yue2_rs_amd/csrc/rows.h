@@ -21,6 +21,10 @@ hipError_t launch_dot_gemm(hipStream_t s, int epi, const GemmArgs& g);
 // rows x heads float2 scratch.  head_dim 64 or 128.
 hipError_t launch_rows_attention(hipStream_t s, const FlashArgs& f, float2* stats, int head_dim);
 
+// The self-tests of yue2_hip_selftest_math numbered 21 to 23: n a multiple of
+// 64, 256 and 512.
+hipError_t launch_rows_selftest(hipStream_t s, int which, const float* in, float* out, size_t n);
+
 // Whether the multi-row path takes n tokens appended to `context` cached
 // ones (the shape allows it and it is the faster way).
 bool rows_supported(const Yue2Model* m, int context, int n);

@@ -980,6 +980,43 @@ hipError_t launch_rows_attention(hipStream_t s, const FlashArgs& f, float2* stat
     return hipGetLastError();
 }
 
+// ---- self-tests --------------------------------------------------------------
+
+// what 21: exp_nonpos elementwise.  22, 23: eight-term products through two
+// 16x16x4 or four 32x32x2 FP32 MFMAs from +0, one wave per group of inputs: A
+// [rows][8], then B [columns][8]; out [rows][columns], of the 32 x 32 form the
+// rows of the group's parity (a sum of -0 as +0).
+__global__ __launch_bounds__(64) void rows_selftest_kernel(int which, const float* in, float* out) {
+    const int lane = threadIdx.x, g = blockIdx.x;
+    if (which == 21) {
+        out[g * 64 + lane] = exp_nonpos(in[g * 64 + lane]);
+    } else if (which == 22) {
+        const float *a = in + (size_t)g * 256, *b = a + 128;
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int k = lane >> 4; k < 8; k += 4) acc = mfma_f32_16(a[(lane & 15) * 8 + k], b[(lane & 15) * 8 + k], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[(size_t)g * 256 + (4 * (lane >> 4) + r) * 16 + (lane & 15)] = acc[r] + 0.0f;
+    } else {
+        const float *a = in + (size_t)g * 512, *b = a + 256;
+        f32x16 acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+        for (int k = lane >> 5; k < 8; k += 2) acc = mfma_f32_32(a[(lane & 31) * 8 + k], b[(lane & 31) * 8 + k], acc);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = acc32_row(lane, r);
+            if ((row & 1) == (g & 1)) out[(size_t)g * 512 + (row >> 1) * 32 + acc32_col(lane)] = acc[r] + 0.0f;
+        }
+    }
+}
+
+hipError_t launch_rows_selftest(hipStream_t s, int which, const float* in, float* out, size_t n) {
+    const size_t group = which == 21 ? 64 : which == 22 ? 256 : 512;
+    if (which < 21 || which > 23 || n % group || n / group < 1 || n / group > 0x7fffffff) return hipErrorInvalidValue;
+    rows_selftest_kernel<<<(unsigned)(n / group), 64, 0, s>>>(which, in, out);
+    return hipGetLastError();
+}
+
 // ---- host --------------------------------------------------------------------
 
 // Rows per pass through the layers: the GEMMs gain nothing from more, and

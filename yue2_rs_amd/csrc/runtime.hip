@@ -906,7 +906,7 @@ extern "C" int32_t yue2_hip_synchronize(void) {
 extern "C" int32_t yue2_hip_selftest_math(int32_t which, const void* in, void* out, size_t n) {
     std::lock_guard<std::recursive_mutex> guard(library_lock());
     if (!device_ready()) return fail(YUE2_ERR_DEVICE, "no gfx950 device");
-    if (which < 0 || which > 20 || !in || !out || (which >= 4 && n % 256 != 0))
+    if (which < 0 || which > 23 || !in || !out || (which >= 4 && n % 256 != 0))
         return fail(YUE2_ERR_ARG, "bad selftest request");
     const size_t elem = which == 1 ? sizeof(double) : sizeof(float);
     void *din = nullptr, *dout = nullptr;
@@ -914,7 +914,9 @@ extern "C" int32_t yue2_hip_selftest_math(int32_t which, const void* in, void* o
     if (e == hipSuccess) e = device_malloc(&dout, n * elem);
     if (e == hipSuccess) e = hipMemcpy(din, in, n * elem, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        if (which >= 19) {
+        if (which >= 21) {
+            e = launch_rows_selftest(nullptr, which, static_cast<const float*>(din), static_cast<float*>(dout), n);
+        } else if (which >= 19) {
             e = launch_sine_selftest(nullptr, static_cast<const float*>(din), static_cast<float*>(dout), n, which == 20);
         } else {
             launch_math_selftest(nullptr, which, din, dout, n);
