@@ -453,7 +453,7 @@ int32_t yue2_hip_model_set_step_kernel(Yue2Model *m, int32_t on);
  * 3B-class prompt in ~20 ms, agreeing with the decode-order prefill within
  * its stated tolerance, not bit for bit -- as the reference's GPU prefill,
  * MPS GEMMs, src/tensor.rs:991-993, differs from its CPU path) or, the
- * default, the decode-order prefill (bit-exact, ~150 ms for that prompt).
+ * default, the decode-order prefill (bit-exact, ~140 ms for that prompt).
  * Returns the setting now in force (1 or 0). */
 int32_t yue2_hip_model_set_prefill(Yue2Model *m, int32_t mfma);
 /* Diagnostics: advance the launch sequence of the model's own workspace (the

@@ -289,9 +289,10 @@ static hipError_t launch_gemm_e(hipStream_t s, const GemmArgs& g) {
     // time: the tile with the least rounds x rows, the smaller ones' rows
     // counted dearer for their extra operand reads per MFMA.  Against the
     // 256-row tile wherever it fills half the CUs and else the 128-row one,
-    // us: 2048 x 5120 x 3072 77 -> 69, 4096 156 -> 137; 3003 x 3072 x 3072 78
-    // -> 66, x 8192 189 -> 166, 6000 156 -> 132 and 371 -> 315; the pair at
-    // 517 x 8192 x 3072 95 -> 76.
+    // us: 2048 x 5120 x 3072 71 -> 64, 4096 150 -> 126; 3003 x 3072 x 3072 72
+    // -> 62, x 8192 175 -> 148, 6000 149 -> 126 and 370 -> 319; the pair at
+    // 517 x 8192 x 3072 93 -> 73; no slower on 40 to 24000 rows of the linears
+    // of four models.
     const int tn = EPI == GEPI_SWIGLU_BF16 ? 128 : 256;
     auto cost = [&](int tm, int weight) {
         const long tiles = (long)((g.N + tn - 1) / tn) * ((g.M + tm - 1) / tm);

@@ -7,9 +7,10 @@
 // of them are fma chains from +0 combined by fixed trees.  The FP32 matrix
 // instructions compute exactly that chain: v_mfma_f32_32x32x2_f32 and
 // v_mfma_f32_16x16x4_f32 return fma(a[k+1], b[k+1], fma(a[k], b[k], c))
-// rounded to nearest even after every step, denormals kept (checked on the
-// device against fmaf over normal, wide-range and denormal operands).  So the
-// order is kept on the matrix cores, at 16 x the rows per weight read.
+// rounded to nearest even after every step, denormals kept (self-tests 22 and 23
+// hold them to the oracle's chain over normal, wide-range and denormal
+// operands).  So the
+// order is kept on the matrix cores, 32 rows to a weight read.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -301,7 +302,7 @@ hipError_t launch_dot_gemm(hipStream_t s, int epi, const GemmArgs& g) {
 // 2048 tokens, 37.3 / 38.4 at 6000, 98.4 / 95.7 at 12000, 244 / 215 at 20000
 // (the block sums of 313 blocks leave the shared statistics one workgroup per
 // CU); a 1B class 6.64 / 6.75, 24.8 / 25.6, 68.5 / 70.2, 108 / 112 at 16000.
-// 517 tokens of the YuE2 shape, per layer: 77 us against 236.
+// 517 tokens of the YuE2 shape, per layer: 81 us against 236.
 //
 // The scores are computed transposed, S^T = K Q^T with 16x16x4 MFMAs: lane l has
 // query l % 16 and, of the block, keys 16 kt + 4 (l / 16) + r.  A score's

@@ -303,18 +303,19 @@ __global__ __launch_bounds__(256, 2) void conv_mfma_kernel(const ConvPlan p) {
 // ---- FP32 convolutions on the BF16 matrix cores ------------------------------
 //
 // Each f32 operand is the exact sum of three BF16 parts (x = x0 + x1 + x2, each
-// the rounding of what is left: 8 + 8 + 8 bits), so x w is the sum of nine
-// BF16 products, of which x1 w2, x2 w1 and x2 w2 are below 2^-26 of it and are
-// left out; six 32x32x16 MFMAs with f32 accumulation replace eight FP32 MFMAs
-// of twice the length each.  Against float64 the six products are three times
-// closer than the FP32 chain (1024 x 1024 outputs: 0.35e-6 against 1.07e-6 at
-// 3584 terms, 0.17e-6 against 0.54e-6 at 896), since sixteen products enter
-// each rounding of the sum.  The split is exact for 2^-100 <= |x| < 2^128 -
-// 2^119 (below, what denormal parts lose is under 2^-126; from there on the
-// first part would be infinite, where a weight's is the largest BF16 instead
-// and an activation's is).  Infinities, NaN and such activations leave the
-// accumulators they enter infinite or NaN, and an output that is not finite is
-// computed again as one FP32 chain (split_chain).
+// the rounding of what is left: 8 + 8 + 8 bits, |x1| up to 2^-8 |x| and |x2| up
+// to 2^-17 |x|), so x w is the sum of nine BF16 products, of which x1 w2, x2 w1
+// (up to 2^-25 of it each) and x2 w2 are left out: 2^-24 together at worst, one
+// FP32 rounding of the product.  Six 32x32x16 MFMAs with f32 accumulation
+// replace eight FP32 MFMAs of twice the length each, and a sum of K products
+// rounds 6 K / 16 times instead of K: against float64 its root-mean-square
+// error is 0.67 to 0.90 of the FP32 fma chain's (K = 32 to 7168), the left-out
+// products' share 0.02 to 0.08 of the chain's.  The split is exact for 2^-100
+// <= |x| < 2^128 - 2^119 (below, what denormal parts lose is under 2^-126; from
+// there on the first part would be infinite, where a weight's is the largest
+// BF16 instead and an activation's is).  Infinities, NaN and such activations
+// leave the accumulators they enter infinite or NaN, and an output that is not
+// finite is computed again as one FP32 chain (split_chain).
 //
 // Tile: TM = 32 MI WM output rows x TN = 32 NJ WN output channels, one tap of
 // 16 input channels per step.  The weights are split at load and laid out as
@@ -327,9 +328,10 @@ __global__ __launch_bounds__(256, 2) void conv_mfma_kernel(const ConvPlan p) {
 //
 // Bound: BF16 MFMA issue at the clock that random operands leave (a plain BF16
 // GEMM's ~1.1 PFLOP/s, so ~190 TFLOP/s of FP32 products).  Measured on the
-// 1920-ratio shape: 7-tap convolutions 174 TFLOP/s (conv_mfma_kernel 108), the
-// 1-tap ones at 128 channels 5 TB/s; a three-minute song in 512-frame tiles
-// 263 -> 163 ms, 37 frames 6.58 -> 3.31 ms.
+// 1920-ratio shape, a 544-frame tile: 7-tap convolutions 175 to 195 TFLOP/s at
+// 128 to 512 channels and 144 at 1024 (conv_mfma_kernel 106 to 112 and 78), the
+// 1-tap ones at 128 channels 3 TB/s; a three-minute song in 512-frame tiles
+// 262 -> 163 ms, 37 frames 6.6 -> 3.2 ms.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -868,7 +870,7 @@ hipError_t run_split(ConvPlan& p, int act, int phases, hipStream_t s) {
         for (int q = 0; q < p.ntaps[ph]; ++q) reach = std::max(reach, p.off[ph][q] - p.off_min[ph]);
     }
     const long tiles = (long)((rows + SplitBig::TM - 1) / SplitBig::TM) * (p.cout_pad / SplitBig::TN) * phases;
-    // half the CUs with a big tile each beat 64 x 64 tiles (song 163 ms;
+    // half the 256 CUs with a big tile each beat 64 x 64 tiles (song 163 ms;
     // 166 from 192 tiles on, 168 from 300), a quarter do not (37 frames 3.62
     // against 3.34 ms)
     const bool big = tiles >= 128;
