@@ -809,25 +809,6 @@ ConvShape conv_shape(const VaeOpHost& op) {
 std::vector<float> conv_slabs(const VaeOpHost& op, const ConvShape& c) {
     std::vector<float> t(c.weights(op.kernel), 0.0f);
     const int nchunks = c.cin_pad / c.chunk;
-    if (c.split) {
-        // [tap][16 inputs][32 outputs][part][lane: output l % 32, inputs 8 (l / 32) ..][8]
-        uint16_t* d = reinterpret_cast<uint16_t*>(t.data());
-        for (int o = 0; o < op.cout; ++o)
-            for (int i = 0; i < op.cin; ++i)
-                for (int j = 0; j < op.kernel; ++j) {
-                    float v = op.w[op.kind == VAE_CONVT ? ((size_t)i * op.cout + o) * op.kernel + j
-                                                        : ((size_t)o * op.cin + i) * op.kernel + j];
-                    const size_t frag = (((size_t)j * nchunks + i / 16) * (c.cout_pad / 32) + o / 32) * 3;
-                    const size_t in = (size_t)((i % 16 / 8) * 32 + o % 32) * 8 + i % 8;
-                    for (int part = 0; part < 3; ++part) {
-                        float r = rb(v);
-                        if (std::isinf(r) && std::isfinite(v)) r = std::copysign(kBf16Max, v);
-                        d[(frag + part) * 512 + in] = bf16_bits(r);
-                        v = std::isfinite(r) ? v - r : 0.0f;
-                    }
-                }
-        return t;
-    }
     for (int o = 0; o < op.cout; ++o)
         for (int i = 0; i < op.cin; ++i)
             for (int j = 0; j < op.kernel; ++j) {
@@ -839,6 +820,59 @@ std::vector<float> conv_slabs(const VaeOpHost& op, const ConvShape& c) {
                 t[dst] = op.w[src];
             }
     return t;
+}
+
+// The weights of a split convolution (checkpoint layout) as operand fragments
+// [tap][16 inputs][32 outputs][part][lane: output l % 32, inputs 8 (l / 32) ..
+// + 7], one thread per lane; outputs past the last one are 0.
+__global__ __launch_bounds__(256) void split_weights_kernel(const float* w, uint16_t* d, int cin, int cout, int kernel,
+                                                            int nblk, int transpose) {
+    const size_t id = (size_t)blockIdx.x * 256 + threadIdx.x, frag = id >> 6;
+    const int lane = threadIdx.x & 63, c16s = cin / 16;
+    const int o = (int)(frag % nblk) * 32 + lane % 32, i0 = (int)(frag / nblk % c16s) * 16 + lane / 32 * 8;
+    const int j = (int)(frag / nblk / c16s);
+    if (j >= kernel) return;
+    uint32_t parts[3][4] = {};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float v = 0.0f;
+        if (o < cout) v = w[transpose ? ((size_t)(i0 + e) * cout + o) * kernel + j : ((size_t)o * cin + i0 + e) * kernel + j];
+#pragma unroll
+        for (int part = 0; part < 3; ++part) {
+            float r = rb(v);
+            if (__builtin_isinf(r) && !__builtin_isinf(v)) r = __builtin_copysignf(kBf16Max, v);
+            parts[part][e / 2] |= (uint32_t)bf16_bits(r) << (e & 1) * 16;
+            v = __builtin_isfinite(r) ? v - r : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+        *reinterpret_cast<uint4*>(d + (frag * 3 + part) * 512 + lane * 8) =
+            make_uint4(parts[part][0], parts[part][1], parts[part][2], parts[part][3]);
+}
+
+// A convolution's weights to dst (shape.weights(kernel) floats) in the layout
+// of its kernel.  The fragments are made on the device: on the host they took
+// longer than all the rest of opening a decoder (the 1920-ratio shape, 84 M
+// weights: 0.74 s against 0.10).
+hipError_t upload_weights(hipStream_t s, const VaeOpHost& op, const ConvShape& c, float* dst) {
+    if (!c.split) {
+        const std::vector<float> slabs = conv_slabs(op, c);
+        return hipMemcpy(dst, slabs.data(), sizeof(float) * slabs.size(), hipMemcpyHostToDevice);
+    }
+    float* raw = nullptr;
+    hipError_t e = device_malloc(&raw, sizeof(float) * op.w.size());
+    if (e == hipSuccess) e = hipMemcpy(raw, op.w.data(), sizeof(float) * op.w.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        const int nblk = c.cout_pad / 32;
+        const size_t threads = (size_t)op.kernel * (op.cin / 16) * nblk * 64;
+        split_weights_kernel<<<(unsigned)((threads + 255) / 256), 256, 0, s>>>(
+            raw, reinterpret_cast<uint16_t*>(dst), op.cin, op.cout, op.kernel, nblk, op.kind == VAE_CONVT);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+    }
+    (void)hipFree(raw);
+    return e;
 }
 
 template <typename K>
@@ -1060,7 +1094,10 @@ extern "C" Yue2Vae* yue2_hip_vae_open(const char* dir) {
             *dst = reinterpret_cast<float*>(base + off);
             e = hipMemcpy(*dst, src.data(), src.size() * sizeof(float), hipMemcpyHostToDevice);
         };
-        if (op.kind == VAE_CONV || op.kind == VAE_CONVT) up(conv_slabs(op, v->shape[k]), ow[k], &v->w[k]);
+        if (op.kind == VAE_CONV || op.kind == VAE_CONVT) {
+            v->w[k] = reinterpret_cast<float*>(base + ow[k]);
+            e = upload_weights(v->stream, op, v->shape[k], v->w[k]);
+        }
         up(op.b, ob[k], &v->b[k]);
         up(op.a, oa[k], &v->a[k]);
         up(op.ib, oi[k], &v->ib[k]);
@@ -1285,14 +1322,13 @@ extern "C" int32_t yue2_hip_selftest_conv(int32_t transpose, int32_t cin, int32_
     const int len = conv_length(op, frames);
     if (len <= 0) return fail(YUE2_ERR_ARG, "bad convolution selftest");
     const ConvShape shape = conv_shape(op);
-    const std::vector<float> slabs = conv_slabs(op, shape);
     float *dx = nullptr, *dw = nullptr, *db = nullptr, *dy = nullptr;
     hipError_t e = device_malloc(&dx, sizeof(float) * (size_t)frames * cin);
-    if (e == hipSuccess) e = device_malloc(&dw, sizeof(float) * slabs.size());
+    if (e == hipSuccess) e = device_malloc(&dw, sizeof(float) * shape.weights(kernel));
     if (e == hipSuccess) e = device_malloc(&db, sizeof(float) * cout);
     if (e == hipSuccess) e = device_malloc(&dy, sizeof(float) * (size_t)len * cout);
     if (e == hipSuccess) e = hipMemcpy(dx, x, sizeof(float) * (size_t)frames * cin, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(dw, slabs.data(), sizeof(float) * slabs.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = upload_weights(nullptr, op, shape, dw);
     if (e == hipSuccess && bias) e = hipMemcpy(db, bias, sizeof(float) * cout, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = run_conv(nullptr, op, shape, dw, bias ? db : nullptr, dx, frames, dy, nullptr, ACT_NONE, nullptr, nullptr,
