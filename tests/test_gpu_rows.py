@@ -141,9 +141,11 @@ def test_norm_fallbacks_counted(shape, step_kernel):
 
 
 # (head_dim, context, rows, position of the id whose value overflows): in the
-# middle of a wave's queries and of a block; in the last row of a block; in
-# the kernels of long contexts, with rows on both sides of the 256th block
+# middle of a wave's queries and of a block; in the last row of a block; a few
+# rows past the 256th block; in the kernels of long contexts, with rows on both
+# sides of it
 @pytest.mark.parametrize("head_dim,context,n,at", [(64, 0, 83, 70), (128, 0, 83, 70), (64, 5, 200, 122), (128, 5, 40, 30),
+                                                   (64, 16400, 40, 30), (128, 16400, 40, 30),
                                                    (64, 15000, 2048, 1400), (128, 15000, 2048, 1400)])
 def test_rows_before_an_infinite_value(gpu, head_dim, context, n, at):
     """A row attends the keys up to its own: what is computed for it does not
