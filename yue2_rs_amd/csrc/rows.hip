@@ -336,6 +336,42 @@ __device__ __forceinline__ void stage_keys(const uint16_t* K, int t, int last, u
     }
 }
 
+// V of block t (keys past last: the last one) through registers, transposed, to
+// LDS by the NT threads of a workgroup: a unit is a key pair x 8 dims.
+template <int D, int NT>
+struct ValueStage {
+    static constexpr int UNITS = kBlockKeys / 2 * (D / 8), PER = (UNITS + NT - 1) / NT;
+    uint4 a[PER], b[PER];
+    __device__ __forceinline__ void load(const uint16_t* V, int t, int last) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int u = threadIdx.x + NT * i, k = t * kBlockKeys + 2 * (u % (kBlockKeys / 2));
+            const int vd = u / (kBlockKeys / 2) * 8;
+            if (UNITS % NT && u >= UNITS) continue;
+            a[i] = ldg4(V + (size_t)min(k, last) * D + vd);
+            b[i] = ldg4(V + (size_t)min(k + 1, last) * D + vd);
+        }
+    }
+    // row = dim, key 16 kt + 4 j + r at 16 j + 4 kt + r (a lane's keys are 16
+    // consecutive halfwords), 16-byte units swizzled
+    __device__ __forceinline__ void store(uint16_t* vt) const {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int u = threadIdx.x + NT * i, vd = u / (kBlockKeys / 2) * 8;
+            if (UNITS % NT && u >= UNITS) continue;
+            const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), at = ((k >> 4) & 1) * 4 + (k & 3);
+            const uint32_t x[4] = {a[i].x, a[i].y, a[i].z, a[i].w}, y[4] = {b[i].x, b[i].y, b[i].z, b[i].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int d = vd + e;
+                const uint32_t w = e & 1 ? (x[e >> 1] >> 16) | (y[e >> 1] & 0xffff0000u)
+                                         : (x[e >> 1] & 0xffffu) | (y[e >> 1] << 16);
+                *reinterpret_cast<uint32_t*>(&vt[d * kBlockKeys + ((unit ^ ((d >> 1) & 7)) << 3) + at]) = w;
+            }
+        }
+    }
+};
+
 // This lane's query values: element 8 c + 4 s + j of query l % 16.
 template <int D>
 __device__ __forceinline__ void load_query(const uint16_t* q, bool in, float (&qf)[D / 8][2]) {
@@ -639,11 +675,7 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_stats_kernel(const Flash
 
 template <int D>
 __global__ __launch_bounds__(kRowsThreads, 2) void rows_pv_kernel(const FlashArgs f, const float2* stats) {
-    constexpr int VU = kBlockKeys / 2 * (D / 8);  // V units: a key pair x 8 dims
-    constexpr int VS = (VU + kRowsThreads - 1) / kRowsThreads;  // units per thread
     __shared__ __align__(16) uint16_t ks[2][kBlockKeys * D];
-    // V transposed: row = dim, key 16 kt + 4 j + r at 16 j + 4 kt + r (a
-    // lane's keys are 16 consecutive halfwords), 16-byte units swizzled
     __shared__ __align__(16) uint16_t vt[2][D * kBlockKeys];
     const RowsQuery r = rows_query(f);
     const int tid = threadIdx.x, lane = tid & 63, j = lane >> 4, last = f.p0 + f.rows - 1;
@@ -657,42 +689,18 @@ __global__ __launch_bounds__(kRowsThreads, 2) void rows_pv_kernel(const FlashArg
     f32x4 o[D / 16], pend[D / 16];
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // this thread's V units
-    uint4 va[VS], vb[VS];
-    auto load_values = [&](int t) {
-#pragma unroll
-        for (int i = 0; i < VS; ++i) {
-            const int u = tid + kRowsThreads * i, k = t * kBlockKeys + 2 * (u % (kBlockKeys / 2)), vd = u / (kBlockKeys / 2) * 8;
-            if (u < VU) {
-                va[i] = ldg4(V + (size_t)min(k, last) * D + vd);
-                vb[i] = ldg4(V + (size_t)min(k + 1, last) * D + vd);
-            }
-        }
-    };
+    ValueStage<D, kRowsThreads> values;
     for (bool exact = false;; exact = true) {
         stage_keys<D, kRowsWaves>(K, 0, last, ks[0]);
-        load_values(0);
+        values.load(V, 0, last);
         for (int t = 0; t < tiles; ++t) {
             const int kb = t * kBlockKeys, buf = t & 1;
-#pragma unroll
-            for (int i = 0; i < VS; ++i) {
-                const int u = tid + kRowsThreads * i, vd = u / (kBlockKeys / 2) * 8;
-                if (u >= VU) continue;
-                const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), in = ((k >> 4) & 1) * 4 + (k & 3);
-                const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, b[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int d = vd + e;
-                    const uint32_t w = e & 1 ? (a[e >> 1] >> 16) | (b[e >> 1] & 0xffff0000u)
-                                             : (a[e >> 1] & 0xffffu) | (b[e >> 1] << 16);
-                    *reinterpret_cast<uint32_t*>(&vt[buf][d * kBlockKeys + ((unit ^ ((d >> 1) & 7)) << 3) + in]) = w;
-                }
-            }
+            values.store(vt[buf]);
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             asm volatile("s_barrier" ::: "memory");  // block t is staged, block t - 1 read by every wave
             if (t + 1 < tiles) {
                 stage_keys<D, kRowsWaves>(K, t + 1, last, ks[buf ^ 1]);
-                load_values(t + 1);
+                values.load(V, t + 1, last);
             }
             const bool live = kb <= r.wave_last;
             f32x4 p[4];
@@ -848,11 +856,10 @@ __global__ __launch_bounds__(kShareThreads, 2) void share_stats_kernel(const Fla
 
 template <int D, bool LONG>
 __global__ __launch_bounds__(kShareThreads, D == 64 && !LONG ? 4 : 2) void share_pv_kernel(const FlashArgs f, const float2* stats) {
-    constexpr int VU = kBlockKeys / 2 * (D / 8), VS = VU / kShareThreads > 0 ? VU / kShareThreads : 1;
     constexpr int DW = D / 16 / kShareWaves;  // 16-dim tiles per wave
-    static_assert(VU % kShareThreads == 0 && DW >= 1, "whole units and tiles");
+    static_assert(DW >= 1, "whole tiles");
     __shared__ __align__(16) uint16_t ks[2][kBlockKeys * D];
-    __shared__ __align__(16) uint16_t vt[2][D * kBlockKeys];  // as in rows_pv_kernel
+    __shared__ __align__(16) uint16_t vt[2][D * kBlockKeys];
     __shared__ __align__(16) f32x4 ps[2][kShareWaves][64];    // p of keys 16 kt + 4 j .. + 3, wave kt's lane
     const int tid = threadIdx.x, lane = tid & 63, j = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.x, g = h / (f.heads / f.kv_heads), q0 = (gridDim.y - 1 - blockIdx.y) * 16;
@@ -868,39 +875,18 @@ __global__ __launch_bounds__(kShareThreads, D == 64 && !LONG ? 4 : 2) void share
     f32x4 o[DW], pend[DW];
 #pragma unroll
     for (int d = 0; d < DW; ++d) o[d] = pend[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    uint4 va[VS], vb[VS];
-    auto load_values = [&](int t) {
-#pragma unroll
-        for (int i = 0; i < VS; ++i) {
-            const int u = tid + kShareThreads * i, k = t * kBlockKeys + 2 * (u % (kBlockKeys / 2));
-            const int vd = u / (kBlockKeys / 2) * 8;
-            va[i] = ldg4(V + (size_t)min(k, last) * D + vd);
-            vb[i] = ldg4(V + (size_t)min(k + 1, last) * D + vd);
-        }
-    };
+    ValueStage<D, kShareThreads> values;
     for (bool exact = false;; exact = true) {
         stage_keys<D, kShareWaves>(K, 0, last, ks[0]);
-        load_values(0);
+        values.load(V, 0, last);
         for (int t = 0; t < tiles; ++t) {
             const int kb = t * kBlockKeys, buf = t & 1;
-#pragma unroll
-            for (int i = 0; i < VS; ++i) {
-                const int u = tid + kShareThreads * i, vd = u / (kBlockKeys / 2) * 8;
-                const int k = 2 * (u % (kBlockKeys / 2)), unit = 2 * ((k >> 2) & 3) + (k >> 5), at = ((k >> 4) & 1) * 4 + (k & 3);
-                const uint32_t a[4] = {va[i].x, va[i].y, va[i].z, va[i].w}, b[4] = {vb[i].x, vb[i].y, vb[i].z, vb[i].w};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int d = vd + e;
-                    const uint32_t w = e & 1 ? (a[e >> 1] >> 16) | (b[e >> 1] & 0xffff0000u)
-                                             : (a[e >> 1] & 0xffffu) | (b[e >> 1] << 16);
-                    *reinterpret_cast<uint32_t*>(&vt[buf][d * kBlockKeys + ((unit ^ ((d >> 1) & 7)) << 3) + at]) = w;
-                }
-            }
+            values.store(vt[buf]);
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             asm volatile("s_barrier" ::: "memory");  // block t is staged; block t - 1's scores and p are read
             if (t + 1 < tiles) {
                 stage_keys<D, kShareWaves>(K, t + 1, last, ks[buf ^ 1]);
-                load_values(t + 1);
+                values.load(V, t + 1, last);
             }
             {
                 // the p of this wave's 16 keys (one tile of a half-block's two: the other is another wave's)
