@@ -1052,10 +1052,9 @@ int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, b
     int32_t* dids = reinterpret_cast<int32_t*>(b.p + o_ids);
     hipStream_t s = m->stream;
     const float eps = cf.rms_norm_eps;
-    // the norms' fallbacks, counted as the token steps of this model count them
-    // (the step kernel leaves out the final norm's)
-    int32_t* fallbacks = &m->ws.st->norm_fallbacks;
-    launch_fill(s, reinterpret_cast<float*>(fallbacks), 1, 0.0f);
+    // the norms' fallbacks are counted as the token steps of this model count
+    // them (the step kernel leaves out the final norm's), and read when asked for
+    int32_t* fallbacks = &m->rows_state->norm_fallbacks;
     hipError_t e = hipMemcpyAsync(dids, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, s);
     for (int p0 = 0; p0 < n && e == hipSuccess; p0 += (int)R) {
         const int rows = std::min((int)R, n - p0), pos = c->length + p0;
@@ -1079,7 +1078,8 @@ int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, b
                 e = launch_dot_gemm(s, GEPI_RESID, GemmArgs{act, I, L.wd, nullptr, I, x, nullptr, H, rows, H, I});
         }
         if (e == hipSuccess && head && p0 + rows == n)
-            if (int rc = enqueue_head(m, m->ws, x + (size_t)(rows - 1) * H, phase, s, 1, !m->step_kernel)) {
+            if (int rc = enqueue_head(m, m->ws, x + (size_t)(rows - 1) * H, phase, s, 1,
+                                      m->step_kernel ? nullptr : m->rows_state)) {
                 (void)hipStreamSynchronize(s);
                 return rc;
             }
@@ -1087,9 +1087,6 @@ int run_rows(Yue2Model* m, Yue2Cache* c, const int32_t* ids, int n, int phase, b
     const hipError_t done = hipStreamSynchronize(s);  // nothing runs over the scratch any more
     m->scratch.trim();
     if (e == hipSuccess) e = done;
-    int32_t taken = 0;
-    if (e == hipSuccess && hipMemcpy(&taken, fallbacks, sizeof(taken), hipMemcpyDeviceToHost) == hipSuccess)
-        m->norm_fallbacks += taken;
     return e == hipSuccess ? YUE2_OK : hip_fail(e, "multi-row forward");
 }
 

@@ -134,7 +134,8 @@ struct Yue2Model {
     bool step_kernel = false;            // decode steps through the persistent kernel (default where supported)
     bool prefill_mfma = false;           // yue2_hip_generate prefills on the matrix cores
     y2::Workspace ws;  // batch-1 workspace of the parity API
-    int norm_fallbacks = 0;
+    int norm_fallbacks = 0;               // of the token steps
+    y2::StepState* rows_state = nullptr;  // in block: counts the multi-row calls' since the model was opened
     y2::NarDev nar;    // loaded by yue2_hip_nar_load
     // The live caches and decoders made on this model.  yue2_hip_model_free
     // detaches them: a decoder's device objects are released, a cache keeps
@@ -163,10 +164,10 @@ bool device_ready();
 int enqueue_step(Yue2Model* m, Workspace& w, const KvView& kv, int rows, bool head, int phase,
                  hipStream_t s);
 // The final norm and the phase's LM head of `rows` rows x (stride hidden)
-// into w.logits (Model::forward_phase's projection, src/model.rs:469-507);
-// count: the final norm's fallbacks are counted.
-int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStream_t s, int rows = 1,
-                 bool count = true);
+// into w.logits (Model::forward_phase's projection, src/model.rs:469-507); the
+// final norm's fallbacks are counted in w.st, or in *count (null: not).
+int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStream_t s, int rows = 1);
+int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStream_t s, int rows, StepState* count);
 // The same step as one persistent kernel when the shape has one (full
 // vocabulary head only); returns 1 when it cannot be used.  sample: the
 // fused sampler's mode (StepCall::sample); the workspace must have been

@@ -291,14 +291,18 @@ int enqueue_step(Yue2Model* m, Workspace& w, const KvView& kv, int rows, bool he
     return enqueue_head(m, w, w.x, phase, s, rows);
 }
 
-int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStream_t s, int rows, bool count) {
+int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStream_t s, int rows) {
+    return enqueue_head(m, w, x, phase, s, rows, w.st);
+}
+
+int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStream_t s, int rows, StepState* count) {
     const Yue2Config& c = m->c;
     const int H = c.hidden_size, V = c.vocab_size;
     const float eps = c.rms_norm_eps;
     hipError_t e;
     // final_norm (src/model.rs:590) runs in the LM-head GEMV prologue.
     if (phase == YUE2_PHASE_NONE) {
-        GemvArgs la{m->lm_head, nullptr, x, w.logits, H, V, V, H, rows, m->final_norm, eps, count ? w.st : nullptr};
+        GemvArgs la{m->lm_head, nullptr, x, w.logits, H, V, V, H, rows, m->final_norm, eps, count};
         if ((e = launch_gemv(s, EPI_STORE, la)) != hipSuccess) return hip_fail(e, "gemv(lm_head)");
         return YUE2_OK;
     }
@@ -308,7 +312,7 @@ int enqueue_head(Yue2Model* m, Workspace& w, const float* x, int phase, hipStrea
     phase_range(phase, &start, &end, &stop);
     launch_fill(s, w.logits, (size_t)rows * V, -INFINITY);
     GemvArgs ra{m->lm_head + (size_t)start * H, nullptr, x, w.logits + start, H, V, end - start, H, rows,
-                m->final_norm, eps, count ? w.st : nullptr};
+                m->final_norm, eps, count};
     if ((e = launch_gemv(s, EPI_STORE, ra)) != hipSuccess) return hip_fail(e, "gemv(lm_head range)");
     GemvArgs sa{m->lm_head + (size_t)stop * H, nullptr, x, w.logits + stop, H, V, 1, H, rows,
                 m->final_norm, eps, nullptr};
@@ -524,6 +528,7 @@ extern "C" Yue2Model* yue2_hip_model_open(const Yue2Config* c, const uint16_t* e
         o.kn = cv.take<float>(D);
         o.post = cv.take<float>(H);
     }
+    const size_t o_rows = cv.take<StepState>(1);
     hipError_t e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         hip_fail(e, "hipStreamCreate");
@@ -610,6 +615,8 @@ extern "C" Yue2Model* yue2_hip_model_open(const Yue2Config* c, const uint16_t* e
     // The layer table in device memory, for the persistent step kernel.
     if (ok && device_malloc(&m->layers_dev, sizeof(LayerDev) * m->layers.size()) != hipSuccess) ok = false;
     up(m->layers_dev, m->layers.data(), sizeof(LayerDev) * m->layers.size());
+    m->rows_state = reinterpret_cast<StepState*>(static_cast<char*>(m->block) + o_rows);
+    if (ok && hipMemset(m->rows_state, 0, sizeof(StepState)) != hipSuccess) ok = false;
     if (ok && (hipDeviceGetAttribute(&m->cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess ||
                m->cus <= 0))
         ok = false;
@@ -668,8 +675,11 @@ extern "C" int32_t yue2_hip_model_advance_sequence(Yue2Model* m, int32_t add) {
 }
 
 extern "C" int32_t yue2_hip_norm_fallbacks(const Yue2Model* m) {
+    std::lock_guard<std::recursive_mutex> guard(library_lock());
     if (!m) return 0;
-    return m->norm_fallbacks;
+    StepState rows{};
+    if (hipMemcpy(&rows, m->rows_state, sizeof(rows), hipMemcpyDeviceToHost) != hipSuccess) rows.norm_fallbacks = 0;
+    return m->norm_fallbacks + rows.norm_fallbacks;
 }
 
 extern "C" Yue2Cache* yue2_hip_cache_new(Yue2Model* m, int32_t capacity) {
